@@ -345,12 +345,18 @@ struct Ctx {
 
 __device__ __forceinline__ float bf2f(uint32_t h) { return __uint_as_float(h << 16); }
 
-// fp32 -> bf16 bits, round to nearest even; NaN -> canonical quiet NaN.
-__device__ __forceinline__ uint32_t f2bf(float f) {
-    const uint32_t u = __float_as_uint(f);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return 0x7fc0u;
-    return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+
+// Two fp32 -> packed bf16 bits (a in the low half), round to nearest even,
+// NaN -> quiet NaN: one v_cvt_pk_bf16_f32 where the integer form takes six
+// operations a value and sits on every stage's chain of dependent steps.
+// Bit-equal to the integer rounding for every fp32 value that is no NaN
+// (all 2^32 compared on the device).
+__device__ __forceinline__ uint32_t f2bf_pair(float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t{a, b}), bf16x2_t));
 }
+__device__ __forceinline__ uint32_t f2bf(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
 
 __device__ __forceinline__ float rbf(float f) { return bf2f(f2bf(f)); }
 
@@ -448,14 +454,15 @@ __device__ __forceinline__ float block_sum(float v, float *red) {
 }
 
 __device__ __forceinline__ float sumsq2(uint32_t x) {
-    const float a = bf2f(x & 0xffffu), b = bf2f(x >> 16);
+    const float a = __uint_as_float(x << 16), b = __uint_as_float(x & 0xffff0000u);
     return a * a + b * b;
 }
 
 // python_vm rms_norm on two packed bf16 values: bf16(w * bf16(x * r)).
 __device__ __forceinline__ uint32_t norm2(uint32_t x, uint32_t w, float r) {
-    const float n0 = rbf(bf2f(x & 0xffffu) * r), n1 = rbf(bf2f(x >> 16) * r);
-    return f2bf(bf2f(w & 0xffffu) * n0) | (f2bf(bf2f(w >> 16) * n1) << 16);
+    const uint32_t n = f2bf_pair(__uint_as_float(x << 16) * r, __uint_as_float(x & 0xffff0000u) * r);
+    return f2bf_pair(__uint_as_float(w << 16) * __uint_as_float(n << 16),
+                     __uint_as_float(w & 0xffff0000u) * __uint_as_float(n & 0xffff0000u));
 }
 
 // ---------------------------------------------------------------------------
@@ -2695,12 +2702,10 @@ struct LmRows {
 
 // ---- opcode 7: Mixtral_RMS_LM_Head  (python_vm.py:321-345) ----------------
 
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-
 // logits[r] += bf16(W[r, cols] . normed[cols]) for a pair of rows at a time:
 // one packed bf16 atomic add per pair (rows are even-aligned).
 __device__ __forceinline__ void lm_atomic_pair(uint16_t *logits, int r, float sa, float sb) {
-    const bf16x2_t v = {__builtin_bit_cast(__bf16, (uint16_t)f2bf(sa)), __builtin_bit_cast(__bf16, (uint16_t)f2bf(sb))};
+    const bf16x2_t v = __builtin_convertvector((f32x2_t{sa, sb}), bf16x2_t);
     __builtin_amdgcn_global_atomic_fadd_v2bf16((__attribute__((address_space(1))) bf16x2_t *)(logits + r), v);
 }
 
@@ -2935,8 +2940,7 @@ __device__ __forceinline__ bool dense_down_rows(kp_c &p, SharedState &sh, u32x4 
         if (lane == 0) {
 #pragma unroll
             for (int i = 0; i < NR; i += 2) {
-                const bf16x2_t v = {__builtin_bit_cast(__bf16, (uint16_t)f2bf(acc[i])),
-                                    __builtin_bit_cast(__bf16, (uint16_t)f2bf(acc[i + 1]))};
+                const bf16x2_t v = __builtin_convertvector((f32x2_t{acc[i], acc[i + 1]}), bf16x2_t);
                 __builtin_amdgcn_global_atomic_fadd_v2bf16(
                     (__attribute__((address_space(1))) bf16x2_t *)(p.hidden + row + i), v);
             }
@@ -3125,10 +3129,10 @@ __device__ __forceinline__ bool dense_lm_head_rows(kp_c &p, SharedState &sh, u32
     rms_to_lds(p, sh, act, a.lm_norm);
     ArgBest wb{0.f, -1, false};  // lane 0: the wave's best stored logit
     rows_matvec<NR, NC>(sh, w, a.lm_head, (size_t)p.H, 0, act, r0, nrows, [&](int r, float sa, float sb) {
-        const uint32_t ba = f2bf(sa), bb = f2bf(sb);
-        st_dev32(a.logits + r, ba | (bb << 16));
-        arg_take(wb, bf2f(ba), r);
-        arg_take(wb, bf2f(bb), r + 1);
+        const uint32_t w2 = f2bf_pair(sa, sb);
+        st_dev32(a.logits + r, w2);
+        arg_take(wb, bf2f(w2), r);
+        arg_take(wb, __uint_as_float(w2 & 0xffff0000u), r + 1);
     });
     drain_and_sync();
     if (p.lm_cand != nullptr) lm_best_merge(sh, wb);
@@ -3174,10 +3178,10 @@ __device__ __forceinline__ bool op_dense_lm_head(kp_c &p, SharedState &sh, u32x4
         aa = wave_sum(aa);
         ab = wave_sum(ab);
         if (lane == 0) {
-            const uint32_t ba = f2bf(aa), bb = f2bf(ab);
-            st_dev32(a.logits + ra, ba | (bb << 16));
-            arg_take(wb, bf2f(ba), ra);
-            arg_take(wb, bf2f(bb), ra + 1);
+            const uint32_t w2 = f2bf_pair(aa, ab);
+            st_dev32(a.logits + ra, w2);
+            arg_take(wb, bf2f(w2), ra);
+            arg_take(wb, __uint_as_float(w2 & 0xffff0000u), ra + 1);
         }
     }
     drain_and_sync();
