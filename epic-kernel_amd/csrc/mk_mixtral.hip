@@ -1798,17 +1798,36 @@ __device__ __forceinline__ bool wait_lanes_ge(kp_c &p, SharedState &sh, const in
     return ok;
 }
 
+// This thread's first 8 norm weights, loaded before the wait on the hidden
+// state (they do not depend on it).
+__device__ __forceinline__ u32x4 norm_ahead(kp_c &p, const uint16_t *w) {
+    u32x4 r = {0u, 0u, 0u, 0u};
+    if ((int)threadIdx.x < (p.H >> 3)) r = reinterpret_cast<const u32x4 *>(w)[threadIdx.x];
+    return r;
+}
+
 // act[0 .. H/8) = bf16(w * bf16(h * 1/sqrt(mean(h^2) + eps))) of the current
 // hidden state (python_vm rms_norm, lat/python_vm.py:50-56).  Ends with a
-// workgroup barrier.
-__device__ __forceinline__ void rms_to_lds(kp_c &p, SharedState &sh, u32x4 *act, const uint16_t *w) {
+// workgroup barrier.  The stage is a chain of round trips, not bytes, so the
+// hidden state is read once: a thread keeps its first 8 elements (all of them
+// for H <= 8 * kThreads) across the sum, and `wa` holds their weights
+// (norm_ahead).
+__device__ __forceinline__ void rms_to_lds(kp_c &p, SharedState &sh, u32x4 *act, const uint16_t *w, u32x4 wa) {
     const int tid = threadIdx.x, nv = p.H >> 3;
-    float ss = 0.f;
-    for (int v = tid; v < nv; v += kThreads) ss += sumsq8(ld_dev128(p.hidden, (uint32_t)v * 16u));
+    u32x4 xa = {0u, 0u, 0u, 0u};
+    if (tid < nv) xa = ld_dev128(p.hidden, (uint32_t)tid * 16u);
+    float ss = sumsq8(xa);
+    for (int v = tid + kThreads; v < nv; v += kThreads) ss += sumsq8(ld_dev128(p.hidden, (uint32_t)v * 16u));
     ss = block_sum(ss, sh.red_ss);
     const float r = 1.0f / sqrtf(ss / (float)p.H + p.eps);
     const u32x4 *w4 = reinterpret_cast<const u32x4 *>(w);
-    for (int v = tid; v < nv; v += kThreads) act[v] = norm8(ld_dev128(p.hidden, (uint32_t)v * 16u), w4[v], r);
+    for (int v = tid; v < nv; v += kThreads) {
+        if (v != tid) {
+            xa = ld_dev128(p.hidden, (uint32_t)v * 16u);
+            wa = w4[v];
+        }
+        act[v] = norm8(xa, wa, r);
+    }
     __syncthreads();
 }
 
@@ -1934,6 +1953,18 @@ __device__ __forceinline__ bool op_qkv(kp_c &p, SharedState &sh, u32x4 *act, ins
     PairAhead pre;
     stamp(tim, MK_TEVENT_FIRST_LOAD);
     const int nc = p.H / kChunkElems;
+    const uint16_t *lnw = a.attn_ln + (size_t)layer * p.H;
+    const u32x4 wa = norm_ahead(p, lnw);
+    // the RoPE factors of this thread's first row, too
+    const int k0 = a.Hq * D, v0 = k0 + a.Hkv * D;
+    auto rope_at = [&](const float *table, int r) { return table[(size_t)p.pos * D + (r & (D - 1))]; };
+    const int rt = r0 + (int)threadIdx.x;
+    const bool ropes = (int)threadIdx.x < nrows && rt < v0;
+    float cs = 0.f, sn = 0.f;
+    if (ropes) {
+        cs = rope_at(a.rope_cos, rt);
+        sn = rope_at(a.rope_sin, rt);
+    }
     pair_ahead_load(pre, wq, (size_t)p.H, 0, nc, r0, nrows);
     // the pairs after the ones loaded ahead go to LDS, after the normed
     // hidden state and the block's outputs, as far as the launch's LDS holds
@@ -1943,7 +1974,7 @@ __device__ __forceinline__ bool op_qkv(kp_c &p, SharedState &sh, u32x4 *act, ins
     stamp(tim, MK_TEVENT_AT_GMEM_WAIT);
     if (!p.late_loads && !wait()) return false;
     stamp(tim, MK_TEVENT_DONE_GMEM_WAIT);
-    rms_to_lds(p, sh, act, a.attn_ln + (size_t)layer * p.H);
+    rms_to_lds(p, sh, act, lnw, wa);
 
     float *rowv = reinterpret_cast<float *>(act + (p.H >> 3));  // the block's outputs, bf16-rounded
     matvec_rows_ahead(
@@ -1954,16 +1985,17 @@ __device__ __forceinline__ bool op_qkv(kp_c &p, SharedState &sh, u32x4 *act, ins
     // RoPE on q and k rows (interleaved pairs (2i, 2i+1) share cos/sin[2i]):
     // y = x * cos + rot(x) * sin in fp32 without contraction, rot(a, b) =
     // (-b, a); then q -> q_post_rope, k/v -> the caches at pos_id.
-    const int k0 = a.Hq * D, v0 = k0 + a.Hkv * D;
     const size_t kv_base = ((size_t)layer * a.T + p.pos) * (size_t)(a.Hkv * D);
     for (int i = threadIdx.x; i < nrows; i += kThreads) {
         const int r = r0 + i;
         float y = rowv[i];
         if (r < v0) {
-            const int d = r % D;
             const float partner = rowv[i ^ 1];
-            const float cs = a.rope_cos[(size_t)p.pos * D + d], sn = a.rope_sin[(size_t)p.pos * D + d];
-            y = __fadd_rn(__fmul_rn(y, cs), __fmul_rn((d & 1) ? partner : -partner, sn));
+            if (r != rt) {
+                cs = rope_at(a.rope_cos, r);
+                sn = rope_at(a.rope_sin, r);
+            }
+            y = __fadd_rn(__fmul_rn(y, cs), __fmul_rn((r & 1) ? partner : -partner, sn));
         }
         const uint32_t bits = f2bf(y);
         if (r < k0)
@@ -2721,11 +2753,12 @@ __device__ __forceinline__ bool lm_head_rows(kp_c &p, SharedState &sh, u32x4 *ac
     u32x4 w[NR][NC];
     if (p.late_loads && !wait_ge(p, sh, bar_at(p, last, 6), p.down_arrivals, c, 7, last)) return false;
     stamp(tim, MK_TEVENT_FIRST_LOAD);
+    const u32x4 wa = norm_ahead(p, a.lm_norm);
     if (wave * NR < nrows) load_rows_upto<NR, NC>(w, a.lm_head, (size_t)p.H, r0 + wave * NR, min(NR, nrows - wave * NR), col0, lane);
     stamp(tim, MK_TEVENT_AT_GMEM_WAIT);
     if (!p.late_loads && !wait_ge(p, sh, bar_at(p, last, 6), p.down_arrivals, c, 7, last)) return false;
     stamp(tim, MK_TEVENT_DONE_GMEM_WAIT);
-    rms_to_lds(p, sh, act, a.lm_norm);
+    rms_to_lds(p, sh, act, a.lm_norm, wa);
     rows_matvec<NR, NC>(sh, w, a.lm_head, (size_t)p.H, col0, act + (col0 >> 3), r0, nrows,
                         [&](int r, float sa, float sb) { lm_atomic_pair(a.logits, r, sa, sb); });
     drain_and_sync();
@@ -2758,7 +2791,7 @@ __device__ __forceinline__ bool op_lm_head(kp_c &p, SharedState &sh, u32x4 *act,
     stamp(tim, MK_TEVENT_AT_GMEM_WAIT);
     if (!wait_ge(p, sh, bar_at(p, last, 6), p.down_arrivals, c, 7, last)) return false;
     stamp(tim, MK_TEVENT_DONE_GMEM_WAIT);
-    rms_to_lds(p, sh, act, a.lm_norm);
+    rms_to_lds(p, sh, act, a.lm_norm, norm_ahead(p, a.lm_norm));
     stamp(tim, MK_TEVENT_FIRST_LOAD);
     // longer reduction blocks: a row pair per item
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -2839,6 +2872,8 @@ __device__ __forceinline__ bool op_dense_upgate(kp_c &p, SharedState &sh, u32x4 
     auto wait = [&] { return wait_ge(p, sh, bar_at(p, layer, 4), p.H / p.oproj_bs, c, 5, layer); };
     if (p.late_loads && !wait()) return false;
     stamp(tim, MK_TEVENT_FIRST_LOAD);
+    const uint16_t *lnw = p.ffn_ln + (size_t)layer * p.H;
+    const u32x4 wa = norm_ahead(p, lnw);
     load_ahead();
     stamp(tim, MK_TEVENT_AT_GMEM_WAIT);
     if (!p.late_loads && !wait()) return false;
@@ -2847,7 +2882,7 @@ __device__ __forceinline__ bool op_dense_upgate(kp_c &p, SharedState &sh, u32x4 
         sh.stage_slot = -1;  // every thread has read it (the wait ends in barriers)
         sh.route_layer = layer;  // this layer's O projection is complete: its residual rows are final
     }
-    rms_to_lds(p, sh, act, p.ffn_ln + (size_t)layer * p.H);
+    rms_to_lds(p, sh, act, lnw, wa);
     for (int it = wave; it < S; it += kWaves) {  // the staged items
         const int k = it / p.expert_bs;
         const int row = __builtin_amdgcn_readfirstlane(ins[3 + k]) * p.expert_bs + it - k * p.expert_bs;
@@ -3122,11 +3157,12 @@ __device__ __forceinline__ bool dense_lm_head_rows(kp_c &p, SharedState &sh, u32
     u32x4 w[NR][NC];
     if (p.late_loads && !wait_ge(p, sh, bar_at(p, last, 6), p.down_arrivals, c, 7, last)) return false;
     stamp(tim, MK_TEVENT_FIRST_LOAD);
+    const u32x4 wa = norm_ahead(p, a.lm_norm);
     if (wave * NR < nrows) load_rows_upto<NR, NC>(w, a.lm_head, (size_t)p.H, r0 + wave * NR, min(NR, nrows - wave * NR), 0, lane);
     stamp(tim, MK_TEVENT_AT_GMEM_WAIT);
     if (!p.late_loads && !wait_ge(p, sh, bar_at(p, last, 6), p.down_arrivals, c, 7, last)) return false;
     stamp(tim, MK_TEVENT_DONE_GMEM_WAIT);
-    rms_to_lds(p, sh, act, a.lm_norm);
+    rms_to_lds(p, sh, act, a.lm_norm, wa);
     ArgBest wb{0.f, -1, false};  // lane 0: the wave's best stored logit
     rows_matvec<NR, NC>(sh, w, a.lm_head, (size_t)p.H, 0, act, r0, nrows, [&](int r, float sa, float sb) {
         const uint32_t w2 = f2bf_pair(sa, sb);
@@ -3165,7 +3201,7 @@ __device__ __forceinline__ bool op_dense_lm_head(kp_c &p, SharedState &sh, u32x4
     stamp(tim, MK_TEVENT_AT_GMEM_WAIT);
     if (!wait_ge(p, sh, bar_at(p, last, 6), p.down_arrivals, c, 7, last)) return false;
     stamp(tim, MK_TEVENT_DONE_GMEM_WAIT);
-    rms_to_lds(p, sh, act, a.lm_norm);
+    rms_to_lds(p, sh, act, a.lm_norm, norm_ahead(p, a.lm_norm));
     stamp(tim, MK_TEVENT_FIRST_LOAD);
     // other hidden sizes: a row pair per item
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
