@@ -128,6 +128,7 @@ constexpr int kChunkElems = 512;  // bf16 columns covered by one wave-wide 16 B/
 constexpr int kMinLdsBytes = 84 * 1024;
 constexpr uint32_t kTicksPerUs = 100;  // s_memrealtime runs at 100 MHz
 constexpr int kCachePolicySc1 = 16;     // buffer-load cache policy: device scope
+constexpr int kCachePolicyNt = MK_NT_LOADS ? 2 : 0;  // non-temporal (weights are read once)
 // Work-sharing scratch (int32): [0] exit counter, then a (cursor, done) pair
 // per instruction slot w * queue_len + q.
 constexpr int kScratchSlotBase = 16;
@@ -712,6 +713,7 @@ __device__ __forceinline__ void dot_pair(const uint16_t *row_a, const uint16_t *
 // first min(nc, 8) chunks, loaded ahead: issued before a wait on inputs that
 // the weights do not depend on, so the weight stream overlaps the wait.
 constexpr int kAheadChunks = 8;
+constexpr int kRingSlots = 4, kRingChunks = 2;  // stream_pairs: 16 loads of 1 KiB in flight per wave
 struct PairAhead {
     u32x4 a[kAheadChunks], b[kAheadChunks];
 };
@@ -729,6 +731,87 @@ __device__ __forceinline__ void pair_ahead_load(PairAhead &r, const uint16_t *ma
             r.a[i] = load_stream(wa + i * 64);
             r.b[i] = load_stream(wb + i * 64);
         }
+}
+
+// A uniform 16-byte-per-lane load of 1 KiB at base + byte_off (base and offset
+// uniform) with the non-temporal policy, or, when `live` is false, no memory
+// access at all: a raw buffer load is range-checked, and a buffer of no
+// records returns zero.  Either way it is one load instruction, so the
+// compiler's count of outstanding loads does not depend on `live`.
+__device__ __forceinline__ u32x4 load_stream_if(const uint16_t *base, uint32_t byte_off, bool live, int lane) {
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t *>(base), (short)0, live ? 0x7fffffff : 0, 0x00020000);
+    return __builtin_amdgcn_raw_buffer_load_b128(r, lane * 16, (int)byte_off, kCachePolicyNt);
+}
+
+// A pair of rows (n chunks of 512 columns each) to be dotted with the LDS
+// vector at x16 (u32x4 index): all fields uniform across the wave.
+struct PairItem {
+    const uint16_t *a, *b;
+    int n, x16, id;
+};
+
+// A wave's stream of row pairs through a ring of S register slots, CH chunks
+// of both rows each (2 S CH loads in flight).  A slot is reloaded with the
+// chunks S slots further on as soon as it has been used, across item
+// boundaries, so the wave's loads in flight never drain between items however
+// few chunks a row has.  next(item) gives the wave's next item (false: none);
+// mid() runs once, after the ring has been filled; done(id, a, b) gets each
+// item's wave-wide sums.  Chunks are added in order, as dot_pair adds them.
+// Bound: HBM for long rows, the per-item arithmetic (sums, SiLU, claims) for
+// short ones.  Opcode 5 against one item's loads at a time (dot_pair), kernel
+// time of an MoE layer: H 2560, F 6656, 16 experts 52.5 -> 49.3 us; H 4096,
+// F 14336 122.4 -> 120.3 us; H 1024, F 3584 26.5 -> 25.7 us; H 512, F 1024
+// (one chunk, one item per wave) 20.1 -> 20.7 us.  Opcode 6 on a ring of four
+// 4-chunk slots was 1 to 8 % slower than its two 7-chunk register sets.
+template <int S, int CH, typename Next, typename Mid, typename Done>
+__device__ __forceinline__ void stream_pairs(const u32x4 *xl, int lane, Next next, Mid mid, Done done) {
+    u32x4 ra[S][CH], rb[S][CH];
+    int x[S], n[S], id[S];  // x < 0: the slot holds nothing; id >= 0: its chunks end that item
+    PairItem cur{nullptr, nullptr, 0, 0, 0};
+    bool more = next(cur);
+    int c = 0;
+    auto load = [&](int k) {
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+            const bool live = more && c + j < cur.n;
+            ra[k][j] = load_stream_if(cur.a, (uint32_t)(c + j) * 1024u, live, lane);
+            rb[k][j] = load_stream_if(cur.b, (uint32_t)(c + j) * 1024u, live, lane);
+        }
+        x[k] = more ? cur.x16 + c * 64 : -1;
+        n[k] = cur.n - c;
+        id[k] = c + CH >= cur.n ? cur.id : -1;
+        c += CH;
+        if (more && c >= cur.n) {
+            more = next(cur);
+            c = 0;
+        }
+    };
+#pragma unroll
+    for (int k = 0; k < S; ++k) load(k);
+    mid();
+    float aa = 0.f, ab = 0.f;
+    // slots fill in order: when slot 0 holds nothing, neither do the others
+    while (x[0] >= 0) {
+#pragma unroll
+        for (int k = 0; k < S; ++k) {
+            if (x[k] >= 0) {
+#pragma unroll
+                for (int j = 0; j < CH; ++j) {
+                    if (j < n[k]) {
+                        const u32x4 v = xl[x[k] + j * 64];
+                        aa = dot8(ra[k][j], v, aa);
+                        ab = dot8(rb[k][j], v, ab);
+                    }
+                }
+                if (id[k] >= 0) {
+                    done(id[k], wave_sum(aa), wave_sum(ab));
+                    aa = ab = 0.f;
+                }
+            }
+            load(k);
+        }
+    }
 }
 
 // Byte offset in the dynamic LDS of the 8 KiB (1 KiB per wave) that the
@@ -786,11 +869,17 @@ __device__ __forceinline__ u32x4 norm8(u32x4 x, u32x4 w, float r) {
 
 __device__ __forceinline__ float sumsq8(u32x4 x) { return sumsq2(x.x) + sumsq2(x.y) + sumsq2(x.z) + sumsq2(x.w); }
 
-// Reduce per-thread router partials to the E logits (+ bias).  Every thread
-// sums the per-wave partials itself, so the logits end up in registers after
-// a single workgroup barrier.
+// A value of lane `l` (uniform), in every lane.
+__device__ __forceinline__ float lane_value(float v, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+
+// Reduce per-thread router partials to the E logits (+ bias): lane e of every
+// wave adds expert e's per-wave partials itself (in wave order), so the
+// logits are in registers after a single workgroup barrier, and the sums of
+// all experts take the time of one.  Returns lane e's logit.
 template <int kE>
-__device__ __forceinline__ void finish_logits(kp_c &p, SharedState &sh, const float *acc, float *logits) {
+__device__ __forceinline__ float finish_logits(kp_c &p, SharedState &sh, const float *acc) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
     for (int e = 0; e < Experts<kE>::kMax; ++e) {
@@ -800,23 +889,19 @@ __device__ __forceinline__ void finish_logits(kp_c &p, SharedState &sh, const fl
         }
     }
     __syncthreads();
+    const int e = lane & (MK_MAX_EXPERTS - 1);
+    float s = 0.f;
 #pragma unroll
-    for (int e = 0; e < Experts<kE>::kMax; ++e) {
-        float s = 0.f;
-        if (Experts<kE>::has(p, e)) {
-#pragma unroll
-            for (int i = 0; i < kWaves; ++i) s += sh.red[e * kWaves + i];
-            s += sh.bias[e];
-        }
-        logits[e] = s;
-    }
+    for (int i = 0; i < kWaves; ++i) s += sh.red[e * kWaves + i];
+    return s + sh.bias[e];
 }
 
-// normed hidden (bf16) -> act[0 .. H/8); router logits -> logits[0 .. E) in
-// every thread.  Reads hidden_states, so it runs after the producer wait.
+// normed hidden (bf16) -> act[0 .. H/8); returns the router logit of expert e
+// in lane e of every wave (e < E).  Reads hidden_states, so it runs after the
+// producer wait.
 template <int kE>
-__device__ __forceinline__ void rms_router(kp_c &p, SharedState &sh, u32x4 *act, int layer, const uint16_t *router,
-                           const RouterRegs<kE> &rr, int32_t *tim, float *logits) {
+__device__ __forceinline__ float rms_router(kp_c &p, SharedState &sh, u32x4 *act, int layer, const uint16_t *router,
+                                            const RouterRegs<kE> &rr, int32_t *tim) {
     const int tid = threadIdx.x;
     const int nv = p.H >> 3;
     float acc[Experts<kE>::kMax];
@@ -856,8 +941,9 @@ __device__ __forceinline__ void rms_router(kp_c &p, SharedState &sh, u32x4 *act,
         }
     }
     stamp(tim, 62);
-    finish_logits<kE>(p, sh, acc, logits);
+    const float logit = finish_logits<kE>(p, sh, acc);
     stamp(tim, 63);
+    return logit;
 }
 
 struct Top2 {
@@ -865,35 +951,42 @@ struct Top2 {
     float p0, p1;
 };
 
-// Top-2 of softmax(logits) in descending order, and the two probabilities.
-// softmax is monotonic, so the pair is chosen on the logits (strict
-// comparison: the lower expert index wins a tie); p_i = exp(l_i - max) / sum
-// as torch.softmax computes it.
+// Top-2 of softmax(logits) in descending order, and the two probabilities;
+// lane e holds expert e's logit.  softmax is monotonic, so the pair is chosen
+// on the logits (strict comparison: the lower expert index wins a tie);
+// p_i = exp(l_i - max) / sum as torch.softmax computes it, each lane taking
+// its own expert's exponential and the sum in expert order.
 template <int kE>
-__device__ __forceinline__ Top2 softmax_top2(kp_c &p, const float *logits) {
+__device__ __forceinline__ Top2 softmax_top2(kp_c &p, float logit) {
+    float l[Experts<kE>::kMax];
+#pragma unroll
+    for (int e = 0; e < Experts<kE>::kMax; ++e) l[e] = Experts<kE>::has(p, e) ? lane_value(logit, e) : 0.f;
     int i0 = 0;
-    float l0 = logits[0];
+    float l0 = l[0];
 #pragma unroll
     for (int e = 1; e < Experts<kE>::kMax; ++e) {
-        if (Experts<kE>::has(p, e) && logits[e] > l0) {
+        if (Experts<kE>::has(p, e) && l[e] > l0) {
             i0 = e;
-            l0 = logits[e];
+            l0 = l[e];
         }
     }
     int i1 = -1;
     float l1 = 0.f;
 #pragma unroll
     for (int e = 0; e < Experts<kE>::kMax; ++e) {
-        if (Experts<kE>::has(p, e) && e != i0 && (i1 < 0 || logits[e] > l1)) {
+        if (Experts<kE>::has(p, e) && e != i0 && (i1 < 0 || l[e] > l1)) {
             i1 = e;
-            l1 = logits[e];
+            l1 = l[e];
         }
     }
+    i0 = __builtin_amdgcn_readfirstlane(i0);
+    i1 = __builtin_amdgcn_readfirstlane(i1);
+    const float ex = expf(logit - l0);
     float s = 0.f;
 #pragma unroll
     for (int e = 0; e < Experts<kE>::kMax; ++e)
-        if (Experts<kE>::has(p, e)) s += expf(logits[e] - l0);
-    return Top2{i0, i1, 1.0f / s, expf(l1 - l0) / s};
+        if (Experts<kE>::has(p, e)) s += lane_value(ex, e);
+    return Top2{i0, i1, 1.0f / s, lane_value(ex, i1) / s};
 }
 
 // ---------------------------------------------------------------------------
@@ -915,13 +1008,15 @@ __device__ __forceinline__ int next_local_pair(SharedState &sh, int lane) {
 }
 
 // silu_out[e][r] = bf16(bf16(silu(bf16 g)) * bf16 u) from the wave sums of
-// the gate and up rows (lane 0 stores).
+// the gate and up rows, stored by every active lane for its own (e, r).
+__device__ __forceinline__ void silu_store(kp_c &p, int e, int r, float ag, float au) {
+    const float g = rbf(ag), u = rbf(au);
+    const float sg = rbf(g / (1.0f + expf(-g)));
+    st_dev16(p.silu + (size_t)e * p.F + r, f2bf(sg * u));
+}
+// The same by lane 0 alone.
 __device__ __forceinline__ void silu_store(kp_c &p, int e, int r, float ag, float au, int lane) {
-    if (lane == 0) {
-        const float g = rbf(ag), u = rbf(au);
-        const float sg = rbf(g / (1.0f + expf(-g)));
-        st_dev16(p.silu + (size_t)e * p.F + r, f2bf(sg * u));
-    }
+    if (lane == 0) silu_store(p, e, r, ag, au);
 }
 
 // One item of opcode 5: row r of the FFN dimension for expert slot j, i.e.
@@ -936,23 +1031,6 @@ __device__ __forceinline__ void upgate_item(kp_c &p, const u32x4 *act, int layer
     float ag = 0.f, au = 0.f;
     dot_pair(p.gate + off, p.up + off, act, act, p.H / kChunkElems, lane, ag, au);
     silu_store(p, e, r, wave_sum(ag), wave_sum(au), lane);
-}
-
-// Item `it` of an opcode-5 instruction when its gate and up rows are the
-// ones this wave staged in LDS (the predicted top-1 expert's row row0 + it,
-// staged by the preceding O projection; the loads have landed once the wave
-// has waited for its own loads).
-__device__ __forceinline__ void upgate_item_staged(kp_c &p, const u32x4 *act, int row0, int e, int it,
-                                                   int wave, int lane) {
-    const int nc = p.H / kChunkElems;
-    const u32x4 *sg = act + p.stage_off16 + (wave - 1) * 2 * nc * 64 + lane, *su = sg + nc * 64;
-    __builtin_amdgcn_s_waitcnt(0);
-    float ag = 0.f, au = 0.f;
-    for (int ch = 0; ch < nc; ++ch) {
-        ag = dot8(sg[ch * 64], act[ch * 64 + lane], ag);
-        au = dot8(su[ch * 64], act[ch * 64 + lane], au);
-    }
-    silu_store(p, e, row0 + it, wave_sum(ag), wave_sum(au), lane);
 }
 
 // Wave-level claim of the next item of an instruction.  Lane 0 issues the
@@ -1083,6 +1161,19 @@ __device__ __forceinline__ void upgate_item_done(kp_c &p, SharedState &sh, int l
     }
 }
 
+// The pooled slots of an opcode-5 run share the first one's times (one stream
+// of items over the same window, so each slot's bytes are spread over it).
+__device__ __forceinline__ void share_pool_times(int32_t *tim, int K) {
+    if (tim == nullptr || threadIdx.x != 0) return;
+    for (int m = 1; m < K; ++m) {
+        int32_t *tm = tim + m * MK_TIMING_SLOTS;
+        for (const int ev : {MK_TEVENT_START, MK_TEVENT_AT_GMEM_WAIT, MK_TEVENT_DONE_GMEM_WAIT, MK_TEVENT_FIRST_LOAD,
+                             MK_TEVENT_DONE_GMEM_STORE})
+            tm[ev] = tim[ev];
+        tm[MK_TEVENT_END] = (int32_t)(uint32_t)__builtin_amdgcn_s_memrealtime();
+    }
+}
+
 // `consumed` returns the queue slots handled: without work sharing, the
 // instructions of the same layer that follow this one in the worker's queue
 // (kMaxMerge at most) run as one pool of items, so the routing is computed
@@ -1198,9 +1289,7 @@ __device__ __forceinline__ bool op_rms_router_upgate(kp_c &p, SharedState &sh, u
     if (!(kSpec && p.late_loads) && !wait()) return false;
     stamp(tim, MK_TEVENT_DONE_GMEM_WAIT);
 
-    float logits[Experts<kE>::kMax];
-    rms_router<kE>(p, sh, act, layer, p.router, rr, tim, logits);
-    const Top2 t = softmax_top2<kE>(p, logits);
+    const Top2 t = softmax_top2<kE>(p, rms_router<kE>(p, sh, act, layer, p.router, rr, tim));
     if constexpr (kSpec) {
         // predicted and selected experts, one byte each (0xff: no prediction)
         if (tim != nullptr && threadIdx.x == 0)
@@ -1228,35 +1317,127 @@ __device__ __forceinline__ bool op_rms_router_upgate(kp_c &p, SharedState &sh, u
             st_dev16(p.sel_score, sc0);
             st_dev16(p.sel_score + 1, sc1);
         }
-        // items complete (and arrive) one wave at a time, and a wave may do
-        // none: every wave's part of the publication completes first
-        drain_and_sync();
+        // where items complete (and arrive) one wave at a time, and a wave
+        // may do none, every wave's part of the publication completes first;
+        // otherwise the stage's own end covers it
+        if (p.work_sharing || p.chunk_ctr != nullptr) drain_and_sync();
     }
     stamp(tim, MK_TEVENT_FIRST_LOAD);
 
-    const int lane = tid & 63, wave = tid >> 6;
-    if (p.work_sharing && sh.pool_n <= kMaxPoolIns) {
-        // Own items first: all but the tail from the LDS counter, the tail
-        // through this instruction's cursor; then the group's leftovers.  No
-        // worker waits for another: whoever completes an instruction's items
-        // arrives for it.
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // the instruction's items this workgroup takes from its LDS counter: all
+    // of the pool's, or with work sharing all but the tail
+    const bool sharing = p.work_sharing && sh.pool_n <= kMaxPoolIns;
+    const int items = 2 * nrows, tail = sharing ? tail_items(p, items) : 0;
+    const int total = sharing ? items - tail : __builtin_amdgcn_readfirstlane(sh.grp_first[K]);
+    // the staged items hold the predicted top-1 expert's rows: usable if the
+    // routing picked it first (items 0 .. nrows-1 are slot 0)
+    const bool from_lds = kSpec && kE > 0 && staged > 0 && wave >= 1 && wave <= staged && wave < nrows &&
+                          wave < total && __builtin_amdgcn_readfirstlane(sh.spec_e[0]) == t.i0;
+    // pooled instruction, expert slot and FFN row of item `it`
+    // (the pool's list sits in LDS, whose round trips would show at every
+    // item: an instruction by itself does not read it)
+    auto locate = [&](int it, int &q, int &j, int &r) {
+        int local = it, nr = nrows, base = row0;
+        q = 0;
+        if (K > 1) {
+            while (q + 1 < K && it >= __builtin_amdgcn_readfirstlane(sh.grp_first[q + 1])) ++q;
+            local = it - __builtin_amdgcn_readfirstlane(sh.grp_first[q]);
+            nr = __builtin_amdgcn_readfirstlane(sh.grp_nrows[q]);
+            base = __builtin_amdgcn_readfirstlane(sh.grp_row0[q]);
+        }
+        j = local >= nr;
+        r = base + (j ? local - nr : local);
+    };
+    const int nc = p.H / kChunkElems, e0 = t.i0, de = t.i1 - t.i0;
+    if constexpr (kE == 8 && !kSpec) {
+        if (p.chunk_ctr != nullptr) {
+            // overlap on: an item is counted as soon as the next one's weights
+            // have been used (its SiLU store has then completed), so that
+            // opcode 6 can start on finished column chunks
+            int pending = -1;
+            for (int it = wave; it < total; it = next_local_item(sh, lane)) {
+                int q, j, r;
+                locate(it, q, j, r);
+                const int e = j ? t.i1 : t.i0;
+                float ag = 0.f, au = 0.f;
+                const size_t off = ((size_t)(layer * p.E + e) * p.F + r) * (size_t)p.H;
+                dot_pair(p.gate + off, p.up + off, act, act, nc, lane, ag, au);
+                ag = wave_sum(ag);
+                au = wave_sum(au);
+                __builtin_amdgcn_s_waitcnt(0);
+                upgate_item_done(p, sh, layer, pending, lane);
+                silu_store(p, e, r, ag, au, lane);
+                pending = q;
+            }
+            __builtin_amdgcn_s_waitcnt(0);
+            upgate_item_done(p, sh, layer, pending, lane);
+            drain_and_sync();
+            stamp(tim, MK_TEVENT_DONE_GMEM_STORE);
+            share_pool_times(tim, K);
+            return true;
+        }
+    }
+    // Waves take items from a workgroup counter in LDS rather than a fixed
+    // stride: the memory pipeline favours older waves, so with a fixed split
+    // the youngest wave ends up finishing its last items alone.  Rows of one
+    // or two chunks are the exception: the claim's LDS round trip would take
+    // as long as the item's own arithmetic.
+    const bool strided = nc <= 2;
+    bool started = from_lds;
+    int last = wave;
+    if (from_lds) __builtin_amdgcn_s_waitcnt(0);  // the staged rows (they landed long ago)
+    auto next = [&](PairItem &m) {
+        const int it = !started ? wave : strided ? last + kWaves : next_local_item(sh, lane);
+        started = true;
+        last = it;
+        if (it >= total) return false;
+        int q, j, r;
+        locate(it, q, j, r);
+        const size_t off = ((size_t)(layer * p.E + e0 + j * de) * p.F + r) * (size_t)p.H;
+        m = PairItem{p.gate + off, p.up + off, nc, 0, 2 * r + j};
+        return true;
+    };
+    // An item's sums wait in one lane of (sg, su, sid) each, and up to 64 items
+    // get their SiLU and their stores at once: the exponential and the
+    // division of one lane would hold up the wave's stream at every item.
+    int mine = 0, held = 0, sid = 0;
+    float sg = 0.f, su = 0.f;
+    auto flush = [&] {
+        if (lane < held) silu_store(p, e0 + (sid & 1) * de, sid >> 1, sg, su);
+        mine += held;
+        held = 0;
+    };
+    auto done = [&](int id, float ag, float au) {
+        const bool hold = lane == held;
+        sg = hold ? ag : sg;
+        su = hold ? au : su;
+        sid = hold ? id : sid;
+        // per-item completion times of waves 0 and 7 (timing record only)
+        if (tim != nullptr && lane == 0 && (wave == 0 || wave == kWaves - 1) && mine + held < 16)
+            tim[64 + (wave ? 16 : 0) + mine + held] = (int32_t)(uint32_t)__builtin_amdgcn_s_memrealtime();
+        if (++held == 64) flush();
+    };
+    auto staged_item = [&] {
+        if (!from_lds) return;
+        const u32x4 *wg = act + p.stage_off16 + (wave - 1) * 2 * nc * 64 + lane, *wu = wg + nc * 64;
+        float ag = 0.f, au = 0.f;
+        for (int ch = 0; ch < nc; ++ch) {
+            ag = dot8(wg[ch * 64], act[ch * 64 + lane], ag);
+            au = dot8(wu[ch * 64], act[ch * 64 + lane], au);
+        }
+        done(2 * (row0 + wave), wave_sum(ag), wave_sum(au));
+    };
+    stream_pairs<kRingSlots, kRingChunks>(act + lane, lane, next, staged_item, done);
+    flush();
+    if (sharing) {
+        // The tail goes through this instruction's cursor; then the group's
+        // leftovers.  No worker waits for another: whoever completes an
+        // instruction's items arrives for it.
         const int self_slot = c.worker * p.queue_len + c.slot;
         int self_k = 0;
         while (self_k < sh.pool_n - 1 && sh.pool_slot[self_k] != self_slot) ++self_k;
         int32_t *cursor = slot_cursor(p, self_slot);
-        const int items = 2 * nrows, tail = tail_items(p, items);
-        // a wave's first item (item `wave`) may be staged in LDS, as in the
-        // static path below
-        const bool from_lds = kSpec && kE > 0 && staged > 0 && wave >= 1 && wave <= staged && wave < nrows &&
-                              __builtin_amdgcn_readfirstlane(sh.spec_e[0]) == t.i0;
-        int mine = 0;
-        for (int it = wave; it < items - tail; it = next_local_item(sh, lane)) {
-            if (kSpec && kE > 0 && mine == 0 && from_lds)
-                upgate_item_staged(p, act, row0, t.i0, it, wave, lane);
-            else
-                upgate_item(p, act, layer, row0, nrows, t.i0, t.i1, it, lane);
-            ++mine;
-        }
         mine += upgate_claimed(p, act, layer, row0, nrows, t.i0, t.i1, items - tail, tail, cursor, lane);
         // wave 0 also carries the owner's extra count
         publish_items(p, cursor + 1, mine + (wave == 0), items, row0, nrows, layer, lane);
@@ -1265,67 +1446,10 @@ __device__ __forceinline__ bool op_rms_router_upgate(kp_c &p, SharedState &sh, u
         drain_and_sync();
         stamp(tim, MK_TEVENT_DONE_GMEM_STORE);
     } else {
-        // Waves take items from a workgroup counter in LDS rather than a
-        // fixed stride: the memory pipeline favours older waves, so with a
-        // fixed split the youngest wave ends up finishing its last items
-        // alone.  An item is counted once the next one's weights have been
-        // used: its SiLU store has then completed (a wait for it costs
-        // nothing there), so no wave stops streaming to publish rows.
-        const int total = __builtin_amdgcn_readfirstlane(sh.grp_first[K]);
-        // the staged items hold the predicted top-1 expert's rows: usable if
-        // the routing picked it first (items 0 .. nrows-1 are slot 0)
-        const bool from_lds = kSpec && kE > 0 && staged > 0 && wave >= 1 && wave <= staged &&
-                              __builtin_amdgcn_readfirstlane(sh.spec_e[0]) == t.i0;
-        int k = 0, pending = -1;
-        for (int it = wave; it < total; ++k) {
-            int q = 0;
-            while (q + 1 < K && it >= __builtin_amdgcn_readfirstlane(sh.grp_first[q + 1])) ++q;
-            const int local = it - __builtin_amdgcn_readfirstlane(sh.grp_first[q]);
-            const int r0 = __builtin_amdgcn_readfirstlane(sh.grp_row0[q]);
-            const int nr = __builtin_amdgcn_readfirstlane(sh.grp_nrows[q]);
-            const int j = local >= nr;
-            const int r = r0 + (j ? local - nr : local);
-            const int e = j ? t.i1 : t.i0;
-            float ag = 0.f, au = 0.f;
-            if (kSpec && kE > 0 && k == 0 && from_lds) {
-                // this wave's own staged rows (its loads have landed: it has
-                // waited for its hidden-state loads since)
-                const int nc = p.H / kChunkElems;
-                const u32x4 *sg = act + p.stage_off16 + (wave - 1) * 2 * nc * 64 + lane, *su = sg + nc * 64;
-                __builtin_amdgcn_s_waitcnt(0);
-                for (int ch = 0; ch < nc; ++ch) {
-                    ag = dot8(sg[ch * 64], act[ch * 64 + lane], ag);
-                    au = dot8(su[ch * 64], act[ch * 64 + lane], au);
-                }
-            } else {
-                const size_t off = ((size_t)(layer * p.E + e) * p.F + r) * (size_t)p.H;
-                dot_pair(p.gate + off, p.up + off, act, act, p.H / kChunkElems, lane, ag, au);
-            }
-            ag = wave_sum(ag);
-            au = wave_sum(au);
-            __builtin_amdgcn_s_waitcnt(0);
-            upgate_item_done(p, sh, layer, pending, lane);
-            silu_store(p, e, r, ag, au, lane);
-            pending = q;
-            // per-item completion times of waves 0 and 7 (timing record only)
-            if (tim != nullptr && lane == 0 && (wave == 0 || wave == kWaves - 1) && k < 16)
-                tim[64 + (wave ? 16 : 0) + k] = (int32_t)(uint32_t)__builtin_amdgcn_s_memrealtime();
-            it = next_local_item(sh, lane);
-        }
-        __builtin_amdgcn_s_waitcnt(0);
-        upgate_item_done(p, sh, layer, pending, lane);
         drain_and_sync();
+        arrive(p, bar_at(p, layer, 5), total / (2 * p.expert_bs));
         stamp(tim, MK_TEVENT_DONE_GMEM_STORE);
-        // the pooled slots share this one's times (one stream of items over
-        // the same window, so each slot's bytes are spread over it)
-        if (tim != nullptr && threadIdx.x == 0)
-            for (int m = 1; m < K; ++m) {
-                int32_t *tm = tim + m * MK_TIMING_SLOTS;
-                for (const int ev : {MK_TEVENT_START, MK_TEVENT_AT_GMEM_WAIT, MK_TEVENT_DONE_GMEM_WAIT,
-                                     MK_TEVENT_FIRST_LOAD, MK_TEVENT_DONE_GMEM_STORE})
-                    tm[ev] = tim[ev];
-                tm[MK_TEVENT_END] = (int32_t)(uint32_t)__builtin_amdgcn_s_memrealtime();
-            }
+        share_pool_times(tim, K);
     }
     return true;
 }
@@ -1588,9 +1712,11 @@ __device__ __forceinline__ bool op_expert_downproj(kp_c &p, SharedState &sh, u32
     }
     // The residual rows this instruction updates: when opcode 5 ran here,
     // the O-projection barrier it waited for has made them final, so they
-    // are read now instead of after the sums (one dependent load less).
+    // are read now instead of after the sums (one dependent load less; as
+    // the aligned pair of rows, because a 16-bit load is followed at once by
+    // its widening, which would wait for the weights in flight too).
     uint32_t hpre = 0;
-    if (known && tid < first_batch) hpre = ld_dev16(p.hidden + row0 + tid);
+    if (known && tid < first_batch) hpre = ld_dev32(p.hidden + ((row0 + tid) & ~1));
 
     stamp(tim, MK_TEVENT_AT_GMEM_WAIT);
     int32_t *ready = bar_at(p, layer, 5);
@@ -1600,10 +1726,11 @@ __device__ __forceinline__ bool op_expert_downproj(kp_c &p, SharedState &sh, u32
     // with ordinary (cache-allocating) loads straight into a scratch corner
     // of LDS; after the wait, their regular loads find them in the
     // Infinity Cache.  Workgroups that arrive after the last producer skip
-    // it.
+    // it, and their poll has been the wait.
+    bool reached = false;
     if (known && p.pf_rounds > 0) {
-        const bool warm = !counter_reached(p, sh, ready, expected);
-        if (warm) {
+        reached = counter_reached(p, sh, ready, expected);
+        if (!reached) {
             __attribute__((address_space(3))) void *sink =
                 (__attribute__((address_space(3))) void *)(act + (lds_prefetch_offset(p) >> 4) + wave * 64);
             for (int m = 1; m <= p.pf_rounds; ++m) {
@@ -1619,7 +1746,7 @@ __device__ __forceinline__ bool op_expert_downproj(kp_c &p, SharedState &sh, u32
             }
         }
     }
-    if (!wait_ge(p, sh, ready, expected, c, 6, layer)) return false;
+    if (!reached && !wait_ge(p, sh, ready, expected, c, 6, layer)) return false;
     stamp(tim, MK_TEVENT_DONE_GMEM_WAIT);
 
     int e0, e1;
@@ -1703,7 +1830,8 @@ __device__ __forceinline__ bool op_expert_downproj(kp_c &p, SharedState &sh, u32
                 d1 += sh.part[(r * 2 + 1) * kMaxSegments + sg];
             }
             uint16_t *hp = p.hidden + row0 + b0 + r;
-            float h = bf2f(known && b0 == 0 ? hpre : ld_dev16(hp));  // r == tid in the first batch
+            // r == tid in the first batch
+            float h = bf2f(known && b0 == 0 ? (hpre >> (16 * ((row0 + r) & 1))) & 0xffffu : ld_dev16(hp));
             h = rbf(h + rbf(s0 * rbf(d0)));
             h = rbf(h + rbf(s1 * rbf(d1)));
             st_dev16(hp, f2bf(h));
@@ -1739,9 +1867,7 @@ __device__ __forceinline__ bool op_predict(kp_c &p, SharedState &sh, u32x4 *act,
         if (!wait_ge(p, sh, bar_at(p, layer - 1, 6), p.down_arrivals, c, 8, layer)) return false;
         stamp(tim, MK_TEVENT_DONE_GMEM_WAIT);
     }
-    float logits[Experts<kE>::kMax];
-    rms_router<kE>(p, sh, act, layer, weights, rr, tim, logits);
-    const Top2 t = softmax_top2<kE>(p, logits);
+    const Top2 t = softmax_top2<kE>(p, rms_router<kE>(p, sh, act, layer, weights, rr, tim));
     if (threadIdx.x == 0) {
         st_dev32(p.pred_idx, (uint32_t)t.i0);
         st_dev32(p.pred_idx + 1, (uint32_t)t.i1);
