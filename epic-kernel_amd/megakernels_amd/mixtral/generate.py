@@ -49,6 +49,12 @@ from .mk import MixtralMK_Interpreter
 from .scheduler import make_dag, make_globals
 
 
+def _own_interpreters():
+    from ..latency.mk import LatencyMK_Interpreter
+
+    return MixtralMK_Interpreter, LatencyMK_Interpreter
+
+
 class MK_Generator:
     def __init__(self, model, interpreter: MixtralMK_Interpreter, schedule: Schedule, barrier_fill_val: int = 0,
                  skip_mk: bool = False, skip_rest: bool = False, device_argmax: bool = True,
@@ -109,6 +115,12 @@ class MK_Generator:
         costs only the kernel's fixed overhead (megakernels/generators.py:118-119)."""
         self.schedule.globs.instructions.zero_()
 
+    def _launch_takes_embed(self) -> bool:
+        """Whether the interpreter is one of the package's own over its own
+        launcher, which runs ``before_launch``."""
+        return (type(self.interpreter) in _own_interpreters()
+                and getattr(self.interpreter.mk_func, "takes_before_launch", False))
+
     def run(self, input_ids: torch.Tensor, pos_id: int) -> torch.Tensor:
         """One step from ``input_ids``; returns the output token (0-d)."""
         return self._step(input_ids, pos_id)
@@ -120,8 +132,17 @@ class MK_Generator:
         view the kernel writes the token into.  ``embed_next``: the launch
         also writes that token's embedding into ``hidden_states``."""
         globs = self.schedule.globs
+        embed = None
         if not embedded and not self.skip_rest:
-            globs.hidden_states.copy_(self.model.embed_tokens[input_ids.reshape(-1)[0]])
+            # indexing by a device token waits for the stream: as late as the
+            # launch allows, so that its checks run while the GPU works
+            def embed():
+                globs.hidden_states.copy_(self.model.embed_tokens[input_ids.reshape(-1)[0]])
+
+            if self.skip_mk or not self._launch_takes_embed():
+                embed()
+                embed = None
+        late = {} if embed is None else {"before_launch": embed}
         if not self._clean:
             self.fill()
             globs.logits.zero_()
@@ -129,7 +150,7 @@ class MK_Generator:
         if self.skip_mk or not self.device_argmax or self.skip_rest:
             self._clean = False
             if not self.skip_mk:
-                self.interpreter.interpret(globs, **self.launch_kwargs)
+                self.interpreter.interpret(globs, **late, **self.launch_kwargs)
             if self.skip_rest:
                 return input_ids.reshape(-1)[0]
             return torch.argmax(globs.logits, dim=-1)
@@ -138,7 +159,7 @@ class MK_Generator:
         self._clean = False
         self.interpreter.interpret(globs, argmax_out=out,
                                    next_embed_weights=self.model.embed_tokens if embed_next else None,
-                                   reset_for_next_launch=self.reset_next, **self.launch_kwargs)
+                                   reset_for_next_launch=self.reset_next, **late, **self.launch_kwargs)
         self._clean = self.reset_next
         return out
 

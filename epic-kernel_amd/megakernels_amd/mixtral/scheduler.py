@@ -446,7 +446,9 @@ def expected_downproj_arrivals(globs: MixtralGlobals) -> int:
 def prefill_oproj_barrier(globs: MixtralGlobals, layer_idx: int = 0) -> None:
     """Mark layer ``layer_idx``'s O-projection as complete so opcode 5 runs
     without the attention prefix."""
-    globs.barriers[layer_idx, Mixtral_OProj.opcode() - 1, 0] = expected_oproj_arrivals(globs)
+    # fill_, not an item assignment, which copies its value from pageable host
+    # memory and so waits for the stream
+    globs.barriers[layer_idx, Mixtral_OProj.opcode() - 1, 0].fill_(expected_oproj_arrivals(globs))
 
 
 class MixtralLatencyScheduleBuilder(ScheduleBuilder):

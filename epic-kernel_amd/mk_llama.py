@@ -24,7 +24,7 @@ import ctypes
 import torch
 
 import mk_mixtral
-from mk_mixtral import MKError, _check, _check_tensor, _error_text, raise_if_failed
+from mk_mixtral import MKError, _check_tensor, _error_text, raise_if_failed
 
 __all__ = ["mk_llama", "mk_llama_3b", "MkLlamaGlobals", "build_llama_struct"]
 
@@ -141,12 +141,15 @@ def build_llama_struct(
 ) -> MkLlamaGlobals:
     """Validate the reference-ordered arguments and fill the C struct;
     ``TypeError``/``ValueError`` before anything reaches the GPU."""
-    _check(isinstance(hidden_states, torch.Tensor), "hidden_states must be a torch.Tensor", TypeError)
+    if not isinstance(hidden_states, torch.Tensor):
+        raise TypeError("hidden_states must be a torch.Tensor")
     dev = hidden_states.device
-    _check(dev.type == "cuda", f"mk_llama needs GPU tensors, hidden_states is on {dev}")
+    if dev.type != "cuda":
+        raise ValueError(f"mk_llama needs GPU tensors, hidden_states is on {dev}")
     bf16 = torch.bfloat16
     _check_tensor("up_weights", up_weights, bf16, dev)
-    _check(up_weights.dim() == 3, "up_weights must be [L, F, H]")
+    if up_weights.dim() != 3:
+        raise ValueError("up_weights must be [L, F, H]")
     L, F, H = up_weights.shape
     _check_tensor("gate_weights", gate_weights, bf16, dev, (L, F, H))
     _check_tensor("down_weights", down_weights, bf16, dev, (L, H, F))
@@ -154,57 +157,73 @@ def build_llama_struct(
     _check_tensor("attn_norm_weights", attn_norm_weights, bf16, dev, (L, H))
     _check_tensor("hidden_states", hidden_states, bf16, dev, (H,))
     _check_tensor("silu_out", silu_out, bf16, dev, (F,))
-    _check(H % 512 == 0, f"hidden size {H} must be a multiple of 512")
-    _check(k_cache.dim() == 4, "k_cache must be [L*B, T, Hkv, D] (batch 1)")
+    if H % 512 != 0:
+        raise ValueError(f"hidden size {H} must be a multiple of 512")
+    if k_cache.dim() != 4:
+        raise ValueError("k_cache must be [L*B, T, Hkv, D] (batch 1)")
     _, T, Hkv, D = k_cache.shape
-    _check(D in (64, 128), f"head_dim must be 64 or 128, got {D}")
+    if D not in (64, 128):
+        raise ValueError(f"head_dim must be 64 or 128, got {D}")
     _check_tensor("attn_lse_intermediates", attn_lse_intermediates, torch.float32, dev)
-    _check(attn_lse_intermediates.dim() == 2, "attn_lse_intermediates must be [Hq, P]")
+    if attn_lse_intermediates.dim() != 2:
+        raise ValueError("attn_lse_intermediates must be [Hq, P]")
     Hq, P = attn_lse_intermediates.shape
-    _check(Hkv > 0 and Hq % Hkv == 0 and 1 <= Hq // Hkv <= 4, f"need Hq / Hkv in 1..4, got {Hq} / {Hkv}")
-    _check((Hq * D) % 512 == 0, f"Hq * head_dim ({Hq * D}) must be a multiple of 512")
+    if not (Hkv > 0 and Hq % Hkv == 0 and 1 <= Hq // Hkv <= 4):
+        raise ValueError(f"need Hq / Hkv in 1..4, got {Hq} / {Hkv}")
+    if (Hq * D) % 512 != 0:
+        raise ValueError(f"Hq * head_dim ({Hq * D}) must be a multiple of 512")
     _check_tensor("qkv_weights", qkv_weights, bf16, dev, (L, (Hq + 2 * Hkv) * D, H))
     _check_tensor("o_weights", o_weights, bf16, dev, (L, H, Hq * D))
     _check_tensor("k_cache", k_cache, bf16, dev, (L, T, Hkv, D))
     _check_tensor("v_cache", v_cache, bf16, dev, (L, T, Hkv, D))
     _check_tensor("rope_cos", rope_cos, torch.float32, dev)
-    _check(rope_cos.dim() == 2 and rope_cos.shape[1] == D and rope_cos.shape[0] >= T, "rope_cos must be [>=T, D]")
+    if not (rope_cos.dim() == 2 and rope_cos.shape[1] == D and rope_cos.shape[0] >= T):
+        raise ValueError("rope_cos must be [>=T, D]")
     _check_tensor("rope_sin", rope_sin, torch.float32, dev, tuple(rope_cos.shape))
     _check_tensor("q_post_rope", q_post_rope, bf16, dev, (Hq * D,))
     _check_tensor("attn_out", attn_out, bf16, dev, (Hq * D,))
     _check_tensor("attn_out_intermediates", attn_out_intermediates, torch.float32, dev, (Hq, P, D))
     _check_tensor("logits", logits, bf16, dev)
-    _check(logits.dim() == 1, "logits must be [V]")
+    if logits.dim() != 1:
+        raise ValueError("logits must be [V]")
     V = logits.numel()
     _check_tensor("lm_head_norm_weights", lm_head_norm_weights, bf16, dev)
-    _check(lm_head_norm_weights.numel() == H, "lm_head_norm_weights must have H elements")
+    if lm_head_norm_weights.numel() != H:
+        raise ValueError("lm_head_norm_weights must have H elements")
     _check_tensor("lm_head_weights", lm_head_weights, bf16, dev, (V, H))
-    _check(0 <= int(pos_id) < T, f"pos_id {pos_id} outside the KV cache ({T} positions)")
+    if not (0 <= int(pos_id) < T):
+        raise ValueError(f"pos_id {pos_id} outside the KV cache ({T} positions)")
     R = int(matvec_reduction_size) if matvec_reduction_size is not None else H
-    _check(R % 512 == 0 and R > 0 and F % R == 0, f"matvec_reduction_size {R} must be a multiple of 512 dividing {F}")
+    if not (R % 512 == 0 and R > 0 and F % R == 0):
+        raise ValueError(f"matvec_reduction_size {R} must be a multiple of 512 dividing {F}")
     if R != F:
-        _check(R // 512 in (1, 2, 4, 8), f"matvec_reduction_size {R} must be F ({F}) or 512, 1024, 2048, 4096")
-        _check(int(down_proj_block_size) % (16 // (R // 512)) == 0,
-               f"down_proj_block_size {down_proj_block_size} must be a multiple of {16 // (R // 512)} "
-               f"(opcode-6 row group for matvec_reduction_size {R})")
+        if R // 512 not in (1, 2, 4, 8):
+            raise ValueError(f"matvec_reduction_size {R} must be F ({F}) or 512, 1024, 2048, 4096")
+        if int(down_proj_block_size) % (16 // (R // 512)) != 0:
+            raise ValueError(f"down_proj_block_size {down_proj_block_size} must be a multiple of {16 // (R // 512)} "
+                             f"(opcode-6 row group for matvec_reduction_size {R})")
     for name, bs, dim, even in (("up_gate_proj_block_size", up_gate_proj_block_size, F, False),
                                 ("down_proj_block_size", down_proj_block_size, H, True),
                                 ("o_proj_block_size", o_proj_block_size, H, True),
                                 ("qkv_block_size", qkv_block_size, D, True),
                                 ("lm_head_block_size", lm_head_block_size, V, True)):
-        _check(int(bs) > 0 and dim % int(bs) == 0 and (not even or int(bs) % 2 == 0),
-               f"{name}={bs} must {'be even and ' if even else ''}divide {dim}")
-    _check(int(attn_kv_block_size) > 0, "attn_kv_block_size must be positive")
+        if not (int(bs) > 0 and dim % int(bs) == 0 and (not even or int(bs) % 2 == 0)):
+            raise ValueError(f"{name}={bs} must {'be even and ' if even else ''}divide {dim}")
+    if int(attn_kv_block_size) <= 0:
+        raise ValueError("attn_kv_block_size must be positive")
     _check_tensor("barriers", Bar, torch.int32, dev)
-    _check(Bar.dim() == 3 and Bar.shape[0] >= L and Bar.shape[1] >= 7 and Bar.shape[2] >= Hq + 2 * Hkv,
-           "barriers must be [L, >=7, >=Hq+2Hkv]")
+    if not (Bar.dim() == 3 and Bar.shape[0] >= L and Bar.shape[1] >= 7 and Bar.shape[2] >= Hq + 2 * Hkv):
+        raise ValueError("barriers must be [L, >=7, >=Hq+2Hkv]")
     _check_tensor("instructions", instructions, torch.int32, dev)
-    _check(instructions.dim() == 3 and instructions.shape[2] == 32, "instructions must be [W, Q, 32]")
+    if not (instructions.dim() == 3 and instructions.shape[2] == 32):
+        raise ValueError("instructions must be [W, Q, 32]")
     W, Q, _ = instructions.shape
-    _check(W > 0 and Q > 0, "empty instruction tensor")
+    if not (W > 0 and Q > 0):
+        raise ValueError("empty instruction tensor")
     if timings is not None:
         _check_tensor("timings", timings, torch.int32, dev, (W, Q, 128))
-    _check(record_timings is False or timings is not None, "record_timings needs a timings tensor")
+    if not (record_timings is False or timings is not None):
+        raise ValueError("record_timings needs a timings tensor")
     if status is not None:
         _check_tensor("status", status, torch.int32, dev, min_numel=mk_mixtral.STATUS_WORDS)
 
@@ -258,18 +277,22 @@ def launch_struct(g: MkLlamaGlobals, device: torch.device, stream=None) -> None:
         raise MKError(rc, _error_text(lib, rc))
 
 
-def mk_llama(*args, stream=None, debug_sync: bool = False, **kwargs):
+def mk_llama(*args, stream=None, debug_sync: bool = False, before_launch=None, **kwargs):
     """Launch one decode step of the dense VM; same positional arguments as
-    the reference binding (``demos/low-latency-llama/llama_3b.cu:26-54``)."""
+    the reference binding (``demos/low-latency-llama/llama_3b.cu:26-54``);
+    ``before_launch`` as in :func:`mk_mixtral.mk_mixtral`."""
     if len(args) != 27:
         raise TypeError(f"mk_llama takes 27 positional arguments, got {len(args)}")
     load_library()
     g = build_llama_struct(*args, **kwargs)
     device = args[16].device
+    if before_launch is not None:
+        before_launch()
     with torch.cuda.device(device):
         launch_struct(g, device, stream)
         if debug_sync:
             raise_if_failed(device)
 
 
+mk_llama.takes_before_launch = True
 mk_llama_3b = mk_llama

@@ -252,20 +252,24 @@ def _ptr(t):
     return None if t is None else ctypes.c_void_p(t.data_ptr())
 
 
-def _check(cond: bool, msg: str, exc=ValueError):
-    if not cond:
-        raise exc(msg)
-
-
 def _check_tensor(name, t, dtype, device, shape=None, min_numel=None):
-    _check(isinstance(t, torch.Tensor), f"{name} must be a torch.Tensor", TypeError)
-    _check(t.dtype == dtype, f"{name} must be {dtype}, got {t.dtype}", TypeError)
-    _check(t.device == device, f"{name} is on {t.device}, expected {device}")
-    _check(t.is_contiguous(), f"{name} must be contiguous")
-    if shape is not None:
-        _check(tuple(t.shape) == tuple(shape), f"{name} has shape {tuple(t.shape)}, expected {tuple(shape)}")
-    if min_numel is not None:
-        _check(t.numel() >= min_numel, f"{name} has {t.numel()} elements, needs >= {min_numel}")
+    # a launch checks some thirty tensors while the GPU may be waiting for it:
+    # one test when all is well, messages only for what is wrong
+    if (isinstance(t, torch.Tensor) and t.dtype == dtype and t.device == device and t.is_contiguous()
+            and (shape is None or t.shape == shape) and (min_numel is None or t.numel() >= min_numel)):
+        return
+    if not isinstance(t, torch.Tensor):
+        raise TypeError(f"{name} must be a torch.Tensor")
+    if t.dtype != dtype:
+        raise TypeError(f"{name} must be {dtype}, got {t.dtype}")
+    if t.device != device:
+        raise ValueError(f"{name} is on {t.device}, expected {device}")
+    if not t.is_contiguous():
+        raise ValueError(f"{name} must be contiguous")
+    if shape is not None and tuple(t.shape) != tuple(shape):
+        raise ValueError(f"{name} has shape {tuple(t.shape)}, expected {tuple(shape)}")
+    if min_numel is not None and t.numel() < min_numel:
+        raise ValueError(f"{name} has {t.numel()} elements, needs >= {min_numel}")
 
 
 def query_device(device=None) -> tuple[int, int]:
@@ -350,18 +354,23 @@ def build_globals_struct(
     Raises ``TypeError``/``ValueError`` for wrong dtypes, devices, layouts or
     inconsistent shapes, before anything reaches the GPU.
     """
-    _check(isinstance(hidden_states, torch.Tensor), "hidden_states must be a torch.Tensor", TypeError)
+    if not isinstance(hidden_states, torch.Tensor):
+        raise TypeError("hidden_states must be a torch.Tensor")
     dev = hidden_states.device
-    _check(dev.type == "cuda", f"mk_mixtral needs GPU tensors, hidden_states is on {dev}")
+    if dev.type != "cuda":
+        raise ValueError(f"mk_mixtral needs GPU tensors, hidden_states is on {dev}")
     bf16 = torch.bfloat16
 
     _check_tensor("expert_gate_weights", expert_gate_weights, bf16, dev)
-    _check(expert_gate_weights.dim() == 3, "expert_gate_weights must be [L*E, F, H]")
+    if expert_gate_weights.dim() != 3:
+        raise ValueError("expert_gate_weights must be [L*E, F, H]")
     LE, F, H = expert_gate_weights.shape
     _check_tensor("ffn_ln_weights", ffn_ln_weights, bf16, dev)
-    _check(ffn_ln_weights.dim() == 2 and ffn_ln_weights.shape[1] == H, "ffn_ln_weights must be [L, H]")
+    if not (ffn_ln_weights.dim() == 2 and ffn_ln_weights.shape[1] == H):
+        raise ValueError("ffn_ln_weights must be [L, H]")
     L = ffn_ln_weights.shape[0]
-    _check(L > 0 and LE % L == 0, f"expert depth {LE} is not a multiple of {L} layers")
+    if not (L > 0 and LE % L == 0):
+        raise ValueError(f"expert depth {LE} is not a multiple of {L} layers")
     E = LE // L
     _check_tensor("expert_up_weights", expert_up_weights, bf16, dev, (LE, F, H))
     _check_tensor("expert_down_weights", expert_down_weights, bf16, dev, (LE, H, F))
@@ -373,28 +382,37 @@ def build_globals_struct(
     k = selected_expert_indices.numel()
     _check_tensor("selected_expert_scores", selected_expert_scores, bf16, dev, (k,))
     _check_tensor("predicted_expert_indices", predicted_expert_indices, torch.int32, dev, (k,))
-    _check(k == 2, f"num_experts_per_tok must be 2, got {k}")
-    _check(2 <= E <= MAX_EXPERTS, f"num_experts must be in [2, {MAX_EXPERTS}], got {E}")
-    _check(H % 512 == 0 and F % 512 == 0, f"hidden ({H}) and intermediate ({F}) sizes must be multiples of 512")
+    if k != 2:
+        raise ValueError(f"num_experts_per_tok must be 2, got {k}")
+    if not (2 <= E <= MAX_EXPERTS):
+        raise ValueError(f"num_experts must be in [2, {MAX_EXPERTS}], got {E}")
+    if not (H % 512 == 0 and F % 512 == 0):
+        raise ValueError(f"hidden ({H}) and intermediate ({F}) sizes must be multiples of 512")
 
     _check_tensor("barriers", Bar, torch.int32, dev)
-    _check(Bar.dim() == 3 and Bar.shape[0] >= L and Bar.shape[1] >= 8, "barriers must be [L, >=8, width]")
+    if not (Bar.dim() == 3 and Bar.shape[0] >= L and Bar.shape[1] >= 8):
+        raise ValueError("barriers must be [L, >=8, width]")
     _check_tensor("instructions", instructions, torch.int32, dev)
-    _check(instructions.dim() == 3 and instructions.shape[2] == 32, "instructions must be [W, Q, 32]")
+    if not (instructions.dim() == 3 and instructions.shape[2] == 32):
+        raise ValueError("instructions must be [W, Q, 32]")
     W, Q, _ = instructions.shape
-    _check(W > 0 and Q > 0, "empty instruction tensor")
+    if not (W > 0 and Q > 0):
+        raise ValueError("empty instruction tensor")
     if timings is not None:
         _check_tensor("timings", timings, torch.int32, dev, (W, Q, 128))
-    _check(record_timings is False or timings is not None, "record_timings needs a timings tensor")
+    if not (record_timings is False or timings is not None):
+        raise ValueError("record_timings needs a timings tensor")
 
     for name, bs, dim in (("expert_proj_block_size", expert_proj_block_size, F),
                           ("down_proj_block_size", down_proj_block_size, H),
                           ("o_proj_block_size", o_proj_block_size, H)):
-        _check(int(bs) > 0 and dim % int(bs) == 0, f"{name}={bs} must divide {dim}")
+        if not (int(bs) > 0 and dim % int(bs) == 0):
+            raise ValueError(f"{name}={bs} must divide {dim}")
 
     if router_bias is not None:
         _check_tensor("router_bias", router_bias, torch.float32, dev, min_numel=LE)
-        _check(router_bias.numel() == LE, f"router_bias must have L*E={LE} elements")
+        if router_bias.numel() != LE:
+            raise ValueError(f"router_bias must have L*E={LE} elements")
     if predictor_weights is not None:
         _check_tensor("predictor_weights", predictor_weights, bf16, dev, (LE, H))
     if status is not None:
@@ -465,15 +483,18 @@ def build_globals_struct(
 def _decode_tail(argmax_out, next_embed_weights, has_lm_head: bool, dev, H: int):
     """Pointers of the optional in-kernel argmax / next-token embedding."""
     if next_embed_weights is not None:
-        _check(argmax_out is not None, "next_embed_weights needs argmax_out")
+        if argmax_out is None:
+            raise ValueError("next_embed_weights needs argmax_out")
         _check_tensor("next_embed_weights", next_embed_weights, torch.bfloat16, dev)
-        _check(next_embed_weights.dim() == 2 and next_embed_weights.shape[1] == H,
-               f"next_embed_weights must be [V, {H}]")
+        if not (next_embed_weights.dim() == 2 and next_embed_weights.shape[1] == H):
+            raise ValueError(f"next_embed_weights must be [V, {H}]")
     if argmax_out is None:
         return None, None
-    _check(has_lm_head, "argmax_out needs the LM head (attention tensors)")
-    _check(isinstance(argmax_out, torch.Tensor) and argmax_out.dtype == torch.int64 and argmax_out.device == dev
-           and argmax_out.numel() >= 1, "argmax_out must be an int64 tensor on the launch device", TypeError)
+    if not has_lm_head:
+        raise ValueError("argmax_out needs the LM head (attention tensors)")
+    if not (isinstance(argmax_out, torch.Tensor) and argmax_out.dtype == torch.int64 and argmax_out.device == dev
+            and argmax_out.numel() >= 1):
+        raise TypeError("argmax_out must be an int64 tensor on the launch device")
     return argmax_out.data_ptr(), None if next_embed_weights is None else next_embed_weights.data_ptr()
 
 
@@ -484,14 +505,19 @@ def _attention_shape(qkv, attn_ln, o_proj, lm_norm, lm_head, k_cache, v_cache, r
     if not (isinstance(qkv, torch.Tensor) and qkv.numel()):
         return None
     bf16 = torch.bfloat16
-    _check(k_cache.dim() == 4, "k_cache must be [L*B, T, Hkv, D] (batch 1)")
+    if k_cache.dim() != 4:
+        raise ValueError("k_cache must be [L*B, T, Hkv, D] (batch 1)")
     LB, T, Hkv, D = k_cache.shape
-    _check(LB == L, f"k_cache has {LB} layer rows, expected {L} (batch 1)")
-    _check(D in (64, 128), f"head_dim must be 64 or 128, got {D}")
+    if LB != L:
+        raise ValueError(f"k_cache has {LB} layer rows, expected {L} (batch 1)")
+    if D not in (64, 128):
+        raise ValueError(f"head_dim must be 64 or 128, got {D}")
     _check_tensor("attn_lse_intermediates", lse_int, torch.float32, dev)
-    _check(lse_int.dim() == 2, "attn_lse_intermediates must be [Hq, P]")
+    if lse_int.dim() != 2:
+        raise ValueError("attn_lse_intermediates must be [Hq, P]")
     Hq, P = lse_int.shape
-    _check(Hkv > 0 and Hq % Hkv == 0 and 1 <= Hq // Hkv <= 4, f"need Hq / Hkv in 1..4, got {Hq} / {Hkv}")
+    if not (Hkv > 0 and Hq % Hkv == 0 and 1 <= Hq // Hkv <= 4):
+        raise ValueError(f"need Hq / Hkv in 1..4, got {Hq} / {Hkv}")
     QKV = (Hq + 2 * Hkv) * D
     _check_tensor("qkv_weights", qkv, bf16, dev, (L, QKV, H))
     _check_tensor("attn_norm_weights", attn_ln, bf16, dev, (L, H))
@@ -499,22 +525,30 @@ def _attention_shape(qkv, attn_ln, o_proj, lm_norm, lm_head, k_cache, v_cache, r
     _check_tensor("k_cache", k_cache, bf16, dev, (L, T, Hkv, D))
     _check_tensor("v_cache", v_cache, bf16, dev, (L, T, Hkv, D))
     _check_tensor("rope_cos", rope_cos, torch.float32, dev, min_numel=T * D)
-    _check(rope_cos.dim() == 2 and rope_cos.shape[1] == D and rope_cos.shape[0] >= T, "rope_cos must be [T, D]")
+    if not (rope_cos.dim() == 2 and rope_cos.shape[1] == D and rope_cos.shape[0] >= T):
+        raise ValueError("rope_cos must be [T, D]")
     _check_tensor("rope_sin", rope_sin, torch.float32, dev, tuple(rope_cos.shape))
     _check_tensor("q_post_rope", q_rope, bf16, dev, (Hq * D,))
     _check_tensor("attn_out", attn_out, bf16, dev, (Hq * D,))
     _check_tensor("attn_out_intermediates", out_int, torch.float32, dev, (Hq, P, D))
     _check_tensor("logits", logits, bf16, dev)
     V = logits.numel()
-    _check(logits.dim() == 1, "logits must be [V]")
+    if logits.dim() != 1:
+        raise ValueError("logits must be [V]")
     _check_tensor("lm_head_norm_weights", lm_norm, bf16, dev, min_numel=H)
-    _check(lm_norm.numel() == H, "lm_head_norm_weights must have H elements")
+    if lm_norm.numel() != H:
+        raise ValueError("lm_head_norm_weights must have H elements")
     _check_tensor("lm_head_weights", lm_head, bf16, dev, (V, H))
-    _check(0 <= pos_id < T, f"pos_id {pos_id} outside the KV cache ({T} positions)")
-    _check(qkv_bs > 0 and D % qkv_bs == 0 and qkv_bs % 2 == 0, f"qkv_block_size {qkv_bs} must be even and divide {D}")
-    _check(kv_bs > 0, "attn_kv_block_size must be positive")
-    _check(lm_bs > 0 and lm_bs % 2 == 0 and V % lm_bs == 0, f"lm_head_block_size {lm_bs} must be even, divide {V}")
-    _check(lm_red % 512 == 0 and lm_red > 0, "lm_head_reduction must be a multiple of 512")
+    if not (0 <= pos_id < T):
+        raise ValueError(f"pos_id {pos_id} outside the KV cache ({T} positions)")
+    if not (qkv_bs > 0 and D % qkv_bs == 0 and qkv_bs % 2 == 0):
+        raise ValueError(f"qkv_block_size {qkv_bs} must be even and divide {D}")
+    if kv_bs <= 0:
+        raise ValueError("attn_kv_block_size must be positive")
+    if not (lm_bs > 0 and lm_bs % 2 == 0 and V % lm_bs == 0):
+        raise ValueError(f"lm_head_block_size {lm_bs} must be even, divide {V}")
+    if not (lm_red % 512 == 0 and lm_red > 0):
+        raise ValueError("lm_head_reduction must be a multiple of 512")
     return qkv_bs, kv_bs, lm_bs, lm_red, Hq, Hkv, D, V, T, P
 
 
@@ -528,15 +562,22 @@ def launch_struct(g: MkMixtralGlobals, device: torch.device, stream=None) -> Non
         raise MKError(rc, _error_text(lib, rc))
 
 
-def mk_mixtral(*args, stream=None, debug_sync: bool = False, **kwargs):
+def mk_mixtral(*args, stream=None, debug_sync: bool = False, before_launch=None, **kwargs):
     """Launch the persistent MoE megakernel; same positional arguments as the
-    reference binding (``demos/mixtral/mixtral.cu:43-93``)."""
+    reference binding (``demos/mixtral/mixtral.cu:43-93``).  ``before_launch``
+    is called once everything is checked, right before the launch: work that
+    has to wait for the GPU goes there, so that the checks run meanwhile."""
     if len(args) != 32:
         raise TypeError(f"mk_mixtral takes 32 positional arguments, got {len(args)}")
     load_library()
     g = build_globals_struct(*args, **kwargs)
     device = args[17].device
+    if before_launch is not None:
+        before_launch()
     with torch.cuda.device(device):
         launch_struct(g, device, stream)
         if debug_sync:
             raise_if_failed(device)
+
+
+mk_mixtral.takes_before_launch = True
