@@ -2373,7 +2373,6 @@ __device__ __forceinline__ bool partial_attn(kp_c &p, attn_c &a, SharedState &sh
 
     stamp(tim, MK_TEVENT_AT_GMEM_STORE);  // wave 0's positions done
     // fold the token slots of the wave (lanes with the same dp) to the wave max
-    const bool packed = G == 16;  // uniform: head dim 128, four slots = the wave's four rows of 16 lanes
 #pragma unroll
     for (int h = 0; h < GQA; ++h) {
         // partners at lane distance 8 (head dim 64 only), 16 and 32
@@ -2385,16 +2384,9 @@ __device__ __forceinline__ bool partial_attn(kp_c &p, attn_c &a, SharedState &sh
         L[h] *= f;
 #pragma unroll
         for (int j = 0; j < 8; ++j) acc[h][j] *= f;
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            const int o = 8 << k;
-            if (o < G) continue;
-            L[h] += lane_xor(L[h], o, lane);
-            if (!packed) {
-#pragma unroll
-                for (int j = 0; j < 8; ++j) acc[h][j] += lane_xor(acc[h][j], o, lane);
-            }
-        }
+        if (G == 8) L[h] += lane_xor(L[h], 8, lane);
+        L[h] += lane_xor(L[h], 16, lane);
+        L[h] += lane_xor(L[h], 32, lane);
         M[h] = mw;
     }
     // per-wave partials to LDS after the ring: m, l [kWaves][GQA], acc [kWaves][GQA][D]
@@ -2408,36 +2400,35 @@ __device__ __forceinline__ bool partial_attn(kp_c &p, attn_c &a, SharedState &sh
             wl[wave * GQA + h] = L[h];
         }
     }
-    if (packed) {
-        // The four rows' acc summed two registers per swap: v_permlane32_swap
-        // of (a_j, a_{j+4}) plus an add leaves a_j in the lower half and
-        // a_{j+4} in the upper (rows 0+2 and 1+3 added); v_permlane16_swap of
-        // (s_j, s_{j+2}) plus an add leaves in row r the whole sum of a_{j+2r}.
-        // Row r of t0, t1 then holds dims dp * 8 + 2r, + 1: every lane
-        // stores two.  Six swaps per head where lane exchanges take sixteen.
+    // The wave's four rows of 16 lanes are summed two registers per swap:
+    // v_permlane32_swap of (a_j, a_{j+4}) plus an add leaves a_j in the lower
+    // half and a_{j+4} in the upper (rows 0+2 and 1+3 added);
+    // v_permlane16_swap of (s_j, s_{j+2}) plus an add leaves in row r the
+    // sums of a_{j+2r}.  At head dim 64 a row holds two token slots, added
+    // last.  Row r then holds dims dp * 8 + 2r, + 1 and stores both: six
+    // swaps per head (and two DPP adds at head dim 64) where lane exchanges
+    // register by register take 16 (24).  Head dim 64, 4 heads: 2.5 us from the
+    // positions to the partials before, 1.3 us after.
+    const int row = lane >> 4;
 #pragma unroll
-        for (int h = 0; h < GQA; ++h) {
-            float s[4];
+    for (int h = 0; h < GQA; ++h) {
+        float s[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[h][j]),
-                                                                __float_as_uint(acc[h][j + 4]), false, false);
-                s[j] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-            }
-            float t[2];
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(s[j]), __float_as_uint(s[j + 2]),
-                                                                false, false);
-                t[j] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-            }
-            *reinterpret_cast<float2 *>(wacc + (wave * GQA + h) * D + dp * 8 + 2 * slot) = make_float2(t[0], t[1]);
+        for (int j = 0; j < 4; ++j) {
+            const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[h][j]), __float_as_uint(acc[h][j + 4]),
+                                                            false, false);
+            s[j] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
         }
-    } else if (slot == 0) {
+        float t[2];
 #pragma unroll
-        for (int h = 0; h < GQA; ++h)
-#pragma unroll
-            for (int j = 0; j < 8; ++j) wacc[(wave * GQA + h) * D + dp * 8 + j] = acc[h][j];
+        for (int j = 0; j < 2; ++j) {
+            const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(s[j]), __float_as_uint(s[j + 2]), false,
+                                                            false);
+            t[j] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+            if (G == 8) t[j] += lane_xor(t[j], 8, lane);
+        }
+        if (G == 16 || (lane & 8) == 0)
+            *reinterpret_cast<float2 *>(wacc + (wave * GQA + h) * D + dp * 8 + 2 * row) = make_float2(t[0], t[1]);
     }
     __syncthreads();
     stamp(tim, 55);  // every wave's partials are in LDS

@@ -46,3 +46,16 @@ def test_moe_stream_sizes(hidden, ffn, experts, workers):
         # fp32 sums in another order than the oracle's flip up to 1.2 % of the
         # residuals at these sizes; a lost rounding point flips over 20 %
         case.run_token(x).assert_ok(min_exact=0.98)
+
+
+@pytest.mark.parametrize("hidden,heads,kv_heads,cached", [
+    (1024, 16, 16, 9),    # head dim 64, one query head per KV head, a partly filled chunk
+    (1024, 16, 8, 64),    # two, exactly one chunk of positions
+    (1536, 24, 8, 65),    # three, one position in the second chunk
+    (1024, 16, 4, 300),   # four, several partitions
+])
+def test_head_dim_64_fold(hidden, heads, kv_heads, cached):
+    """The token slots of a wave fold in packed pairs of registers."""
+    case = LlamaCase(LlamaConfig(1, hidden, 512, heads, kv_heads, 64), seed=cached, prefill=cached, steps=1)
+    case.step(3)
+    _check(case, f"head dim 64, {heads} / {kv_heads} heads, {cached} cached")
