@@ -4125,9 +4125,9 @@ int mk_llama_launch(const mk_llama_globals *g, void *stream) {
     const size_t stage_items = stage_limit(
         lds_cap > stage_off ? std::min((size_t)MK_STAGE_ITEMS, (lds_cap - stage_off) / stage_item) : 0, g->late_loads);
     if (stage_items > 0) lds = std::max(lds, stage_off + stage_items * stage_item);
-    // scratch: the work-claim slots, then the exit argmax's candidates (2
-    // ints per workgroup), then the spread counters
-    const size_t cand = kScratchSlotBase + 2 * (size_t)g->num_workers * (size_t)g->queue_len;
+    // scratch: the exit argmax's candidates (2 ints per workgroup; a dense
+    // launch has no work-claim slots), then the spread counters
+    const size_t cand = kScratchSlotBase;
     const SpreadLayout sp = spread_layout(cand + 2 * (size_t)g->num_workers, g->num_layers, g->bar_ops,
                                           kSpreadDenseOps);
     rc = ensure_scratch(st, sp.end);
@@ -4140,9 +4140,11 @@ int mk_llama_launch(const mk_llama_globals *g, void *stream) {
     kp.spread_rows = (int32_t)sp.rows;
     kp.spread_stride = (int32_t)sp.stride;
     kp.spread_ops = sp.ops;
-    // the last workgroup zeroes the claim slots and the candidates (after
-    // the exit argmax has read them): every launch starts from zeroed scratch
-    kp.scratch_clear = (int32_t)(cand + 2 * (size_t)g->num_workers - kScratchSlotBase);
+    // the last workgroup zeroes the candidates (after the exit argmax has
+    // read them): a later Mixtral launch takes them for claim slots.  With the
+    // claim slots of every instruction in front of them, as the work-sharing
+    // launches have, the exit zeroed 400 KB by itself at 28 layers.
+    kp.scratch_clear = g->argmax_out != nullptr ? (int32_t)(2 * g->num_workers) : 0;
     kp.instructions = g->instructions;
     kp.timings = g->record_timings ? g->timings : nullptr;
     kp.bar = g->barriers;
@@ -4312,7 +4314,8 @@ static int launch_mixtral(const mk_mixtral_globals *g, void *stream, bool noallo
     kp.spread_rows = (int32_t)sp.rows;
     kp.spread_stride = (int32_t)sp.stride;
     kp.spread_ops = sp.ops;
-    kp.scratch_clear = (int32_t)(cursors + chunks);
+    // only work sharing uses the cursors, only the overlap the chunk counters
+    kp.scratch_clear = (int32_t)(g->work_sharing || overlap ? cursors + chunks : 0);
     kp.instructions = g->instructions;
     kp.timings = g->record_timings ? g->timings : nullptr;
     kp.bar = g->barriers;

@@ -59,3 +59,29 @@ def test_head_dim_64_fold(hidden, heads, kv_heads, cached):
     case = LlamaCase(LlamaConfig(1, hidden, 512, heads, kv_heads, 64), seed=cached, prefill=cached, steps=1)
     case.step(3)
     _check(case, f"head dim 64, {heads} / {kv_heads} heads, {cached} cached")
+
+
+def test_dense_launches_leave_claim_slots_zero():
+    """A dense launch's argmax candidates share the library's scratch with a
+    work-sharing Mixtral launch's claim slots: the latter's results are the
+    same before and after one."""
+    import torch
+
+    from megakernels_amd.latency.synthetic import LLAMA_TINY, make_synthetic_llama
+    from megakernels_amd.mixtral.generate import MK_Generator
+    from megakernels_amd.mixtral.synthetic import TINY, make_synthetic_mixtral
+
+    dense = MK_Generator.build(make_synthetic_llama(LLAMA_TINY, "cuda", 1, kv_positions=12, prefill=8), 8,
+                               debug_sync=True)
+    moe = MK_Generator.build(make_synthetic_mixtral(TINY, "cuda", 1, full=True, kv_positions=12, prefill=8), 8,
+                             debug_sync=True, reset_next=False)
+    token = torch.tensor([[3]], device="cuda")
+    seen = []
+    for _ in range(3):
+        moe.run(token, 8)
+        g = moe.schedule.globs
+        seen.append((g.logits.clone(), g.hidden_states.clone(), g.barriers.clone()))
+        dense.run(token, 8)
+    for later in seen[1:]:
+        for a, b in zip(seen[0], later):
+            assert torch.equal(a, b)
