@@ -61,6 +61,15 @@ def test_head_dim_64_fold(hidden, heads, kv_heads, cached):
     _check(case, f"head dim 64, {heads} / {kv_heads} heads, {cached} cached")
 
 
+@pytest.mark.parametrize("hidden,vocab", [(1024, 16), (1024, 16 * 300), (1536, 16 * 256 * 5 + 16), (512, 32)])
+def test_dense_lm_head_rows(hidden, vocab):
+    """LM-head items of two rows up to the register limit, a row count that
+    the item does not divide, and the fallback for one-chunk rows."""
+    case = LlamaCase(LlamaConfig(1, hidden, 512, hidden // 64, hidden // 128, vocab), seed=vocab, prefill=5, steps=1)
+    case.step(3)
+    _check(case, f"LM head {vocab} x {hidden}")
+
+
 def test_dense_launches_leave_claim_slots_zero():
     """A dense launch's argmax candidates share the library's scratch with a
     work-sharing Mixtral launch's claim slots: the latter's results are the
