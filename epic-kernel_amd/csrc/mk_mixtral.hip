@@ -756,16 +756,20 @@ struct PairItem {
 // chunks S slots further on as soon as it has been used, across item
 // boundaries, so the wave's loads in flight never drain between items however
 // few chunks a row has.  next(item) gives the wave's next item (false: none);
-// mid() runs once, after the ring has been filled; done(id, a, b) gets each
-// item's wave-wide sums.  Chunks are added in order, as dot_pair adds them.
+// ready() runs once the ring has been filled (false: the stream is given up,
+// and so is its result); mid() once, after MID rounds of the ring; done(id, a,
+// b) gets each item's wave-wide sums.  Chunks are added in order, as dot_pair
+// adds them.
 // Bound: HBM for long rows, the per-item arithmetic (sums, SiLU, claims) for
 // short ones.  Opcode 5 against one item's loads at a time (dot_pair), kernel
 // time of an MoE layer: H 2560, F 6656, 16 experts 52.5 -> 49.3 us; H 4096,
 // F 14336 122.4 -> 120.3 us; H 1024, F 3584 26.5 -> 25.7 us; H 512, F 1024
 // (one chunk, one item per wave) 20.1 -> 20.7 us.  Opcode 6 on a ring of four
-// 4-chunk slots was 1 to 8 % slower than its two 7-chunk register sets.
-template <int S, int CH, typename Next, typename Mid, typename Done>
-__device__ __forceinline__ void stream_pairs(const u32x4 *xl, int lane, Next next, Mid mid, Done done) {
+// 4-chunk slots was 1 to 8 % slower than its two 7-chunk register sets; the
+// LM heads on this ring (16 loads in flight where their items have up to 24)
+// gained nothing at vocab 32000 and 128256 and lost 2 % of a two-layer step.
+template <int S, int CH, int MID, typename Next, typename Ready, typename Mid, typename Done>
+__device__ __forceinline__ bool stream_pairs(const u32x4 *xl, int lane, Next next, Ready ready, Mid mid, Done done) {
     u32x4 ra[S][CH], rb[S][CH];
     int x[S], n[S], id[S];  // x < 0: the slot holds nothing; id >= 0: its chunks end that item
     PairItem cur{nullptr, nullptr, 0, 0, 0};
@@ -789,7 +793,9 @@ __device__ __forceinline__ void stream_pairs(const u32x4 *xl, int lane, Next nex
     };
 #pragma unroll
     for (int k = 0; k < S; ++k) load(k);
-    mid();
+    if (!ready()) return false;
+    bool before = MID > 0;  // mid() is still to come
+    if (!before) mid();
     float aa = 0.f, ab = 0.f;
     // slots fill in order: when slot 0 holds nothing, neither do the others
     while (x[0] >= 0) {
@@ -811,7 +817,13 @@ __device__ __forceinline__ void stream_pairs(const u32x4 *xl, int lane, Next nex
             }
             load(k);
         }
+        if (MID > 0 && before) {
+            mid();
+            before = false;
+        }
     }
+    if (MID > 0 && before) mid();
+    return true;
 }
 
 // Byte offset in the dynamic LDS of the 8 KiB (1 KiB per wave) that the
@@ -1428,7 +1440,7 @@ __device__ __forceinline__ bool op_rms_router_upgate(kp_c &p, SharedState &sh, u
         }
         done(2 * (row0 + wave), wave_sum(ag), wave_sum(au));
     };
-    stream_pairs<kRingSlots, kRingChunks>(act + lane, lane, next, staged_item, done);
+    stream_pairs<kRingSlots, kRingChunks, 0>(act + lane, lane, next, [] { return true; }, staged_item, done);
     flush();
     if (sharing) {
         // The tail goes through this instruction's cursor; then the group's
@@ -2966,83 +2978,87 @@ __device__ __forceinline__ bool op_dense_upgate(kp_c &p, SharedState &sh, u32x4 
         report_error(p, MK_ERR_BAD_INSTRUCTION, c, 5, layer, n, nblocks);
         return false;
     }
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int items = n * p.expert_bs, nc = p.H / kChunkElems;
     // items [0, S) staged in LDS: by the preceding opcode 4 (which left
     // sh.stage_slot / sh.stage_n set before its barriers), else here
     const bool pre_staged = __builtin_amdgcn_readfirstlane(sh.stage_slot) == c.slot;
     const int S = pre_staged ? __builtin_amdgcn_readfirstlane(sh.stage_n)
                              : stage_dense_upgate(p, sh, act, ins, c.slot, layer, false);
-    if (threadIdx.x == 0) sh.next_item = S + kWaves;
-    // each wave's first item from HBM (its gate and up rows) is loaded
-    // before the wait: the weights do not depend on it (issued after the
-    // wait instead, to stream while the staged items are computed, it
-    // measured 7 % slower per decode step)
-    const int ia = S + wave;
-    PairAhead pre;
-    auto load_ahead = [&]() {
-        if (ia < items) {
-            const int k = ia / p.expert_bs;
-            const int row = __builtin_amdgcn_readfirstlane(ins[3 + k]) * p.expert_bs + ia - k * p.expert_bs;
-            const size_t off = ((size_t)layer * p.F + row) * (size_t)p.H;
-            const u32x4 *wg = reinterpret_cast<const u32x4 *>(p.gate + off) + lane;
-            const u32x4 *wu = reinterpret_cast<const u32x4 *>(p.up + off) + lane;
-#pragma unroll
-            for (int i = 0; i < kAheadChunks; ++i)
-                if (i < nc) {
-                    pre.a[i] = load_stream(wg + i * 64);
-                    pre.b[i] = load_stream(wu + i * 64);
-                }
-        }
+    // The other items stream from HBM through each wave's ring, which is
+    // filled before the wait: the weights do not depend on it (issued after
+    // the wait instead, to stream while the staged items are computed, the
+    // first items measured 7 % slower per decode step).  The items that the
+    // fill reaches are dealt in turn, the later ones come from the LDS
+    // counter (as in the MoE's opcode 5, rows of one or two chunks excepted).
+    // Against one item ahead and then one item's loads at a time, kernel time:
+    // eight 3B layers with the LM head 559.7 -> 556.4 us, one layer of H 1536,
+    // F 2048 39.2 -> 38.7 us, two-layer step of H 1024 63.9 -> 63.5 us; one 3B
+    // layer 59.9 -> 59.8 us (no difference).
+    const int dealt = kRingSlots / ((nc + kRingChunks - 1) / kRingChunks) + 1;
+    if (threadIdx.x == 0) sh.next_item = S + dealt * kWaves;
+    const bool strided = nc <= 2;
+    int turn = 0;
+    auto row_of = [&](int it) {
+        const int k = it / p.expert_bs;
+        return __builtin_amdgcn_readfirstlane(ins[3 + k]) * p.expert_bs + it - k * p.expert_bs;
+    };
+    auto next = [&](PairItem &m) {
+        const int it = strided || turn < dealt ? S + turn * kWaves + wave : next_local_item(sh, lane);
+        ++turn;
+        if (it >= items) return false;
+        const int row = row_of(it);
+        const size_t off = ((size_t)layer * p.F + row) * (size_t)p.H;
+        m = PairItem{p.gate + off, p.up + off, nc, 0, row};
+        return true;
     };
     auto wait = [&] { return wait_ge(p, sh, bar_at(p, layer, 4), p.H / p.oproj_bs, c, 5, layer); };
     if (p.late_loads && !wait()) return false;
     stamp(tim, MK_TEVENT_FIRST_LOAD);
     const uint16_t *lnw = p.ffn_ln + (size_t)layer * p.H;
     const u32x4 wa = norm_ahead(p, lnw);
-    load_ahead();
-    stamp(tim, MK_TEVENT_AT_GMEM_WAIT);
-    if (!p.late_loads && !wait()) return false;
-    stamp(tim, MK_TEVENT_DONE_GMEM_WAIT);
-    if (threadIdx.x == 0) {
-        sh.stage_slot = -1;  // every thread has read it (the wait ends in barriers)
-        sh.route_layer = layer;  // this layer's O projection is complete: its residual rows are final
-    }
-    rms_to_lds(p, sh, act, lnw, wa);
-    for (int it = wave; it < S; it += kWaves) {  // the staged items
-        const int k = it / p.expert_bs;
-        const int row = __builtin_amdgcn_readfirstlane(ins[3 + k]) * p.expert_bs + it - k * p.expert_bs;
-        const u32x4 *sg = act + p.stage_off16 + (2 * it) * nc * 64 + lane;
-        const u32x4 *su = sg + nc * 64;
-        float ag = 0.f, au = 0.f;
-        for (int ch = 0; ch < nc; ++ch) {
-            ag = dot8(sg[ch * 64], act[ch * 64 + lane], ag);
-            au = dot8(su[ch * 64], act[ch * 64 + lane], au);
+    auto ready = [&] {
+        stamp(tim, MK_TEVENT_AT_GMEM_WAIT);
+        if (!p.late_loads && !wait()) return false;
+        stamp(tim, MK_TEVENT_DONE_GMEM_WAIT);
+        if (threadIdx.x == 0) {
+            sh.stage_slot = -1;  // every thread has read it (the wait ends in barriers)
+            sh.route_layer = layer;  // this layer's O projection is complete: its residual rows are final
         }
-        silu_store(p, 0, row, wave_sum(ag), wave_sum(au), lane);
-    }
-    if (ia < items) {  // the item loaded ahead
-        const int k = ia / p.expert_bs;
-        const int row = __builtin_amdgcn_readfirstlane(ins[3 + k]) * p.expert_bs + ia - k * p.expert_bs;
-        float ag = 0.f, au = 0.f;
-#pragma unroll
-        for (int i = 0; i < kAheadChunks; ++i)
-            if (i < nc) {
-                ag = dot8(pre.a[i], act[i * 64 + lane], ag);
-                au = dot8(pre.b[i], act[i * 64 + lane], au);
+        rms_to_lds(p, sh, act, lnw, wa);
+        return true;
+    };
+    // sums wait in one lane each, up to 64 items get their SiLU at once (as in
+    // the MoE's opcode 5)
+    int held = 0, srow = 0;
+    float sg = 0.f, su = 0.f;
+    auto flush = [&] {
+        if (lane < held) silu_store(p, 0, srow, sg, su);
+        held = 0;
+    };
+    auto done = [&](int row, float ag, float au) {
+        const bool hold = lane == held;
+        sg = hold ? ag : sg;
+        su = hold ? au : su;
+        srow = hold ? row : srow;
+        if (++held == 64) flush();
+    };
+    // The staged items are computed once the ring has been through its first
+    // round, so that its next items' loads are in flight meanwhile.
+    auto staged_items = [&] {
+        for (int it = wave; it < S; it += kWaves) {
+            const u32x4 *wg = act + p.stage_off16 + (2 * it) * nc * 64 + lane;
+            const u32x4 *wu = wg + nc * 64;
+            float ag = 0.f, au = 0.f;
+            for (int ch = 0; ch < nc; ++ch) {
+                ag = dot8(wg[ch * 64], act[ch * 64 + lane], ag);
+                au = dot8(wu[ch * 64], act[ch * 64 + lane], au);
             }
-        if (nc > kAheadChunks) {
-            const size_t off = ((size_t)layer * p.F + row) * (size_t)p.H + kAheadChunks * kChunkElems;
-            dot_pair(p.gate + off, p.up + off, act + kAheadChunks * 64, act + kAheadChunks * 64, nc - kAheadChunks,
-                     lane, ag, au);
+            done(row_of(it), wave_sum(ag), wave_sum(au));
         }
-        silu_store(p, 0, row, wave_sum(ag), wave_sum(au), lane);
-    }
-    for (int it = next_local_item(sh, lane); it < items; it = next_local_item(sh, lane)) {
-        const int k = it / p.expert_bs;
-        const int row = __builtin_amdgcn_readfirstlane(ins[3 + k]) * p.expert_bs + it - k * p.expert_bs;
-        upgate_item(p, act, layer, row, 1, 0, 0, 0, lane);
-    }
+    };
+    if (!stream_pairs<kRingSlots, kRingChunks, 1>(act + lane, lane, next, ready, staged_items, done)) return false;
+    flush();
     drain_and_sync();
     arrive(p, bar_at(p, layer, 5), n);
     stamp(tim, MK_TEVENT_DONE_GMEM_STORE);

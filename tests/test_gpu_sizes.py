@@ -48,6 +48,23 @@ def test_moe_stream_sizes(hidden, ffn, experts, workers):
         case.run_token(x).assert_ok(min_exact=0.98)
 
 
+@pytest.mark.parametrize("hidden,ffn,workers", [
+    (512, 512, None),    # one chunk per row, every item staged
+    (1024, 4608, 10),    # two chunks, 58 items per wave and instruction
+    (1536, 2048, 12),    # three chunks: half-filled ring slots, three items dealt
+    (2560, 2048, 16),    # five chunks: the counter's items begin inside the ring
+    (3072, 1024, 11),    # six chunks, a last round of fewer items than waves
+    (4608, 1536, 7),     # nine chunks: an item longer than the ring
+])
+@pytest.mark.parametrize("late", [False, True])
+def test_dense_stream_sizes(hidden, ffn, workers, late):
+    """Dense opcode 5's staged items and row stream at the ends of the ring."""
+    case = LlamaCase(LlamaConfig(1, hidden, ffn, hidden // 128, hidden // 256, 64), seed=hidden, prefill=12, steps=1,
+                     workers=workers)
+    case.step(7, late_loads=late)
+    _check(case, f"dense up/gate {ffn} x {hidden}")
+
+
 @pytest.mark.parametrize("hidden,heads,kv_heads,cached", [
     (1024, 16, 16, 9),    # head dim 64, one query head per KV head, a partly filled chunk
     (1024, 16, 8, 64),    # two, exactly one chunk of positions
