@@ -766,8 +766,8 @@ struct PairItem {
 // F 14336 122.4 -> 120.3 us; H 1024, F 3584 26.5 -> 25.7 us; H 512, F 1024
 // (one chunk, one item per wave) 20.1 -> 20.7 us.  Opcode 6 on a ring of four
 // 4-chunk slots was 1 to 8 % slower than its two 7-chunk register sets; the
-// LM heads on this ring (16 loads in flight where their items have up to 24)
-// gained nothing at vocab 32000 and 128256 and lost 2 % of a two-layer step.
+// LM heads on this ring (16 or 24 loads in flight) lost 0.7 % of eight 3B
+// layers and 2 % of a two-layer step.
 template <int S, int CH, int MID, typename Next, typename Ready, typename Mid, typename Done>
 __device__ __forceinline__ bool stream_pairs(const u32x4 *xl, int lane, Next next, Ready ready, Mid mid, Done done) {
     u32x4 ra[S][CH], rb[S][CH];
