@@ -44,15 +44,13 @@ import time
 
 import torch
 
+from ..latency.mk import LatencyMK_Interpreter
 from ..scheduler import Schedule, assign_to_sms, group_rows_by_xcd, tensorize_instructions
 from .mk import MixtralMK_Interpreter
 from .scheduler import make_dag, make_globals
 
-
-def _own_interpreters():
-    from ..latency.mk import LatencyMK_Interpreter
-
-    return MixtralMK_Interpreter, LatencyMK_Interpreter
+# the methods known to pass ``before_launch`` on to the launcher
+_OWN_INTERPRET = (MixtralMK_Interpreter.interpret, LatencyMK_Interpreter.interpret)
 
 
 class MK_Generator:
@@ -89,7 +87,6 @@ class MK_Generator:
         ``globals_kwargs`` to its ``make_globals`` (block sizes, partition
         policy)."""
         if hasattr(model.stacked_params, "gate_proj"):
-            from ..latency.mk import LatencyMK_Interpreter
             from ..latency.scheduler import make_dag as dag_fn
             from ..latency.scheduler import make_globals as globals_fn
 
@@ -116,10 +113,16 @@ class MK_Generator:
         self.schedule.globs.instructions.zero_()
 
     def _launch_takes_embed(self) -> bool:
-        """Whether the interpreter is one of the package's own over its own
-        launcher, which runs ``before_launch``."""
-        return (type(self.interpreter) in _own_interpreters()
-                and getattr(self.interpreter.mk_func, "takes_before_launch", False))
+        """Whether ``interpret`` and the launcher under it are the package's
+        own: a method or a launcher in their place may not know
+        ``before_launch``, or expect the embedding to be there (a wrapped
+        launcher carries the attribute of the one it wraps, hence the
+        identity).  A launch on a stream the caller names stays behind the
+        copy, too."""
+        mk_func = getattr(self.interpreter, "mk_func", None)
+        return (getattr(self.interpreter.interpret, "__func__", None) in _OWN_INTERPRET
+                and mk_func is not None and getattr(mk_func, "takes_before_launch", None) is mk_func
+                and "stream" not in self.launch_kwargs)
 
     def run(self, input_ids: torch.Tensor, pos_id: int) -> torch.Tensor:
         """One step from ``input_ids``; returns the output token (0-d)."""

@@ -294,5 +294,5 @@ def mk_llama(*args, stream=None, debug_sync: bool = False, before_launch=None, *
             raise_if_failed(device)
 
 
-mk_llama.takes_before_launch = True
+mk_llama.takes_before_launch = mk_llama  # itself: a wrapper that copies attributes is another function
 mk_llama_3b = mk_llama

@@ -580,4 +580,4 @@ def mk_mixtral(*args, stream=None, debug_sync: bool = False, before_launch=None,
             raise_if_failed(device)
 
 
-mk_mixtral.takes_before_launch = True
+mk_mixtral.takes_before_launch = mk_mixtral  # itself: a wrapper that copies attributes is another function
