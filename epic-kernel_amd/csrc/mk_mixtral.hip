@@ -150,8 +150,8 @@ constexpr int32_t kSpreadDenseOps = (1 << 3) | (1 << 4) | (1 << 5) | (1 << 6);
 constexpr int32_t kSpreadMixtralOps = (1 << 3) | (1 << 4) | (1 << 5) | (1 << 6);
 constexpr int32_t kSpreadMoeOps = 0;
 constexpr int kPoolGroup = MK_POOL_GROUP;
-constexpr int kMaxPoolIns = 64;  // opcode-5 instructions per (layer, group) that can be shared
 constexpr int kPoolWindow = 8;  // queue slots per group member pool_scan_near looks at
+constexpr int kMaxPoolIns = kPoolGroup * kPoolWindow;  // opcode-5 instructions a group can share
 static_assert(kMaxPoolIns <= 64, "one lane per group instruction");
 constexpr int kRowBatchLds = 64;  // rows per opcode-6 batch (partial sums in LDS)
 constexpr int kMaxSegments = 10;  // column segments per opcode-6 row (F <= 10 * 7 * 512)
@@ -330,7 +330,7 @@ struct SharedState {
     // (-1: none)
     int ostage_slot;
     // opcode 5 over consecutive instructions of one layer (kMaxMerge at
-    // most): first FFN row, rows, first pooled item, finished items
+    // most): first FFN row, rows, first pooled item, finished items (overlap)
     int grp_row0[kMaxMerge], grp_nrows[kMaxMerge], grp_first[kMaxMerge + 1], grp_done[kMaxMerge];
     int ready_mask;  // opcode 6: column groups whose SiLU rows are complete
 };
@@ -1134,7 +1134,7 @@ __device__ __forceinline__ int upgate_claimed(kp_c &p, const u32x4 *act, int lay
 // have completed).  The owner's report carries one extra count, so an
 // instruction completes only after its owner has also published the routing
 // (for the block-0 instruction); the report that reaches items + 1 arrives
-// for the instruction's rows on the layer and chunk counters.
+// for the instruction's rows on the layer counter.
 __device__ __forceinline__ void publish_items(kp_c &p, int32_t *done, int n, int items, int row0,
                                               int nrows, int layer, int lane) {
     if (n <= 0) return;
@@ -1173,22 +1173,20 @@ __device__ __forceinline__ void steal_upgate(kp_c &p, const SharedState &sh, con
     }
 }
 
-// Count a finished item of pooled instruction k (lane 0; the wave's SiLU
-// stores of it have completed).  The item that completes the instruction
-// arrives for its blocks on the layer counter and, with the overlap on, adds
-// its rows to the column-chunk counters.
+// Overlap on: count a finished item of pooled instruction k (lane 0; the
+// wave's SiLU stores of it have completed).  The item that completes the
+// instruction arrives for its blocks on the layer counter and adds its rows
+// to the column-chunk counters.
 __device__ __forceinline__ void upgate_item_done(kp_c &p, SharedState &sh, int layer, int k, int lane) {
     if (lane != 0 || k < 0) return;
     const int r0 = sh.grp_row0[k], n = sh.grp_nrows[k];
     if (atomicAdd(&sh.grp_done[k], 1) + 1 != 2 * n) return;
     arrive_add(p, bar_at(p, layer, 5), n / p.expert_bs);
-    if (p.chunk_ctr != nullptr) {
-        int32_t *cc = p.chunk_ctr + (size_t)layer * (p.F / kChunkElems);
-        for (int r = r0; r < r0 + n;) {
-            const int ch = r / kChunkElems, e = min(r0 + n, (ch + 1) * kChunkElems);
-            __hip_atomic_fetch_add(cc + ch, e - r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            r = e;
-        }
+    int32_t *cc = p.chunk_ctr + (size_t)layer * (p.F / kChunkElems);
+    for (int r = r0; r < r0 + n;) {
+        const int ch = r / kChunkElems, e = min(r0 + n, (ch + 1) * kChunkElems);
+        __hip_atomic_fetch_add(cc + ch, e - r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        r = e;
     }
 }
 
@@ -1258,21 +1256,14 @@ __device__ __forceinline__ bool op_rms_router_upgate(kp_c &p, SharedState &sh, u
                     sh.grp_row0[k] = st_k[k] * p.expert_bs;
                     sh.grp_nrows[k] = nb_k[k] * p.expert_bs;
                     sh.grp_first[k] = first;
-                    sh.grp_done[k] = 0;
+                    if constexpr (kE == 8 && !kSpec) {
+                        if (p.chunk_ctr != nullptr) sh.grp_done[k] = 0;
+                    }
                     first += 2 * nb_k[k] * p.expert_bs;
                 }
             }
             sh.grp_first[K] = first;
         }
-    } else if (threadIdx.x == 0) {
-        // work sharing: a pool of this instruction alone, which the static
-        // path below uses when the group has more instructions than the
-        // shared pool can list
-        sh.grp_row0[0] = start * p.expert_bs;
-        sh.grp_nrows[0] = nb * p.expert_bs;
-        sh.grp_first[0] = 0;
-        sh.grp_first[1] = 2 * nb * p.expert_bs;
-        sh.grp_done[0] = 0;
     }
     consumed = K;
     auto wait = [&] { return wait_ge(p, sh, bar_at(p, layer, 4), p.H / p.oproj_bs, c, 5, layer); };
@@ -1363,7 +1354,7 @@ __device__ __forceinline__ bool op_rms_router_upgate(kp_c &p, SharedState &sh, u
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // the instruction's items this workgroup takes from its LDS counter: all
     // of the pool's, or with work sharing all but the tail
-    const bool sharing = p.work_sharing && sh.pool_n <= kMaxPoolIns;
+    const bool sharing = p.work_sharing;
     const int items = 2 * nrows, tail = sharing ? tail_items(p, items) : 0;
     const int total = sharing ? items - tail : __builtin_amdgcn_readfirstlane(sh.grp_first[K]);
     // the staged items hold the predicted top-1 expert's rows: usable if the
@@ -3484,9 +3475,9 @@ __device__ __forceinline__ void zero_words(uint32_t *p, size_t n) {
     for (size_t i = head + nv * 4 + threadIdx.x; i < n; i += kThreads) p[i] = 0u;
 }
 
-// Exit protocol: the last workgroup out (failed or not) zeroes the
-// work-sharing counters for the next launch, after the decode-driver tail
-// when one was asked for.  Every other workgroup has finished all of its
+// Exit protocol: the last workgroup out (failed or not) zeroes the scratch
+// that the launch used for the next one, after the decode-driver tail when one
+// was asked for.  Every other workgroup has finished all of its
 // scratch accesses before it increments the counter.
 __device__ __forceinline__ void kernel_exit(kp_c &p, SharedState &sh) {
     if (p.lm_cand != nullptr && threadIdx.x == 0) {
@@ -3534,7 +3525,8 @@ __device__ __forceinline__ void kernel_exit(kp_c &p, SharedState &sh) {
                 if ((a.V & 1) && threadIdx.x == 0) a.logits[a.V - 1] = 0;
             }
         }
-        // work-sharing cursors, then the column-chunk counters
+        // Mixtral: work-sharing cursors, then the column-chunk counters; dense:
+        // the argmax candidates
         zero_words(reinterpret_cast<uint32_t *>(p.scratch + kScratchSlotBase), (size_t)p.scratch_clear);
         drain_and_sync();
         if (threadIdx.x == 0) __hip_atomic_store(p.scratch, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -162,11 +162,11 @@ def test_work_sharing(config, workers, mode):
 
 def test_work_sharing_more_instructions_than_the_pool():
     """Work sharing on a schedule whose groups hold more opcode-5
-    instructions than the shared pool lists (one instruction per block,
+    instructions than one pool lists (one instruction per block,
     interleaved: about 45 per worker, ~358 per group of 8 workers at 20
-    workers): every worker then takes the static path for its own
-    instructions, whose item bookkeeping must be set up under work sharing
-    too."""
+    workers, of which a pool lists the at most 64 near one queue depth):
+    owners finish alone what no one near them lists, and every instruction
+    arrives once."""
     case = MoECase(C1, seed=19, workers=20, mode="zz", moe_overlap=True, ln_weight_std=0.1)
     per_worker = (case.g_gpu.instructions[:, :, 0] == 5).sum(dim=1)
     assert int(per_worker[:8].sum()) > 64
