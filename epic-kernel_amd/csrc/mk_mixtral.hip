@@ -770,6 +770,22 @@ struct PairItem {
     int n, x16, id;
 };
 
+// next() calls while a ring is filled from items of nc chunks each: one ahead
+// of the first slot, one after each slot that ends an item.
+template <int S, int CH>
+__device__ __forceinline__ int ring_fill_items(int nc) {
+    int calls = 1, c = 0;
+#pragma unroll
+    for (int k = 0; k < S; ++k) {
+        c += CH;
+        if (c >= nc) {
+            ++calls;
+            c = 0;
+        }
+    }
+    return calls;
+}
+
 // A wave's stream of row pairs through a ring of S register slots, CH chunks
 // of both rows each (2 S CH loads in flight).  A slot is reloaded with the
 // chunks S slots further on as soon as it has been used, across item
@@ -779,6 +795,9 @@ struct PairItem {
 // and so is its result); mid() once, after MID rounds of the ring; done(id, a,
 // b) gets each item's wave-wide sums.  Chunks are added in order, as dot_pair
 // adds them.
+// While the ring is filled (before ready()), next() is called ring_fill_items
+// times, less where the items run out: a caller whose counter is set only by
+// a barrier in ready() deals that many items itself.
 // Bound: HBM for long rows, the per-item arithmetic (sums, SiLU, claims) for
 // short ones.  Opcode 5 against one item's loads at a time (dot_pair), kernel
 // time of an MoE layer: H 2560, F 6656, 16 experts 52.5 -> 49.3 us; H 4096,
@@ -3010,7 +3029,7 @@ __device__ __forceinline__ bool op_dense_upgate(kp_c &p, SharedState &sh, u32x4 
     // eight 3B layers with the LM head 559.7 -> 556.4 us, one layer of H 1536,
     // F 2048 39.2 -> 38.7 us, two-layer step of H 1024 63.9 -> 63.5 us; one 3B
     // layer 59.9 -> 59.8 us (no difference).
-    const int dealt = kRingSlots / ((nc + kRingChunks - 1) / kRingChunks) + 1;
+    const int dealt = ring_fill_items<kRingSlots, kRingChunks>(nc);
     if (threadIdx.x == 0) sh.next_item = S + dealt * kWaves;
     const bool strided = nc <= 2;
     int turn = 0;
