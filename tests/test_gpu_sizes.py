@@ -5,10 +5,12 @@ chunk counts.  Against the CPU oracle, at the repository's bar (max-abs-rel
 
 import pytest
 
+from full_harness import FullCase
 from llama_harness import LlamaCase
 from megakernels_amd.latency.synthetic import LlamaConfig
 from megakernels_amd.mixtral.synthetic import MoEConfig
-from moe_harness import MoECase, draw_tokens
+from megakernels_amd.trace import T_FIRST_USE, T_PREDICTION
+from moe_harness import MoECase, draw_tokens, max_abs_rel
 
 pytestmark = pytest.mark.gpu
 TOL = 2e-2
@@ -111,3 +113,47 @@ def test_dense_launches_leave_claim_slots_zero():
     for later in seen[1:]:
         for a, b in zip(seen[0], later):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("hidden,ffn,experts,workers", [
+    (512, 4096, 3, None),     # one chunk per row, items only in the tail
+    (1536, 4608, 8, 40),      # three chunks, most items ahead of the tail
+    (2560, 1536, 16, 20),     # five
+    (4608, 1024, 8, 33),      # nine: an item longer than the ring
+])
+def test_moe_stream_sizes_shared(hidden, ffn, experts, workers):
+    """The row stream ahead of a work-sharing instruction's claimed tail."""
+    case = MoECase(MoEConfig(1, hidden, ffn, 8, 2, experts, 2, 64), seed=hidden + experts, workers=workers,
+                   ln_weight_std=0.1)
+    for x in draw_tokens(case.cpu_model, 2, margin=1e-2):
+        case.run_token(x, work_sharing=True).assert_ok(min_exact=0.98)
+
+
+@pytest.mark.parametrize("hidden,heads", [(1024, 8), (1536, 12), (2560, 20)])
+@pytest.mark.parametrize("sharing", [False, True])
+def test_predicted_rows_staged_in_lds(hidden, heads, sharing):
+    """A wave's first opcode-5 item comes from LDS where the O projection
+    staged the predicted expert's rows: dealt items after it (two chunks per
+    row), claimed ones (three and five: half-filled ring slots).  The record
+    says that rows were staged and their expert was picked."""
+    # workers without a partition wait at the O projection from the start:
+    # those stage.  16 rows of each expert per worker, so that half of the
+    # items lie ahead of a work-sharing instruction's tail
+    case = FullCase(MoEConfig(1, hidden, 4096, heads, heads // 4, 8, 2, 64), seed=hidden, prefill=600, steps=8,
+                    stop_after_op="downproj", predictor_sigma=1e-4, generate_on_device=True)
+    g, r = case.g_gpu, case.g_cpu
+    used = 0
+    for token in range(3, 9):
+        g.timings.zero_()
+        case.step(token, work_sharing=sharing, record_timings=True)
+        t = g.timings[g.instructions[:, :, 0] == 5].cpu()
+        first = (t[:, T_PREDICTION] & 0xFF) == ((t[:, T_PREDICTION] >> 16) & 0xFF)
+        used += int(((t[:, T_FIRST_USE] != 0) & first).sum())
+        err = case.errors()
+        idx = r.selected_expert_indices.long()
+        assert case.indices()[0] == case.indices()[1]
+        err["silu"] = max_abs_rel(g.expert_silu_out.cpu()[idx], r.expert_silu_out[idx])
+        err["normed"] = max_abs_rel(g.router_normed_hidden, r.router_normed_hidden)
+        print(f"[staged {hidden}] used {used} " + " ".join(f"{k} {v:.2e}" for k, v in err.items()), flush=True)
+        assert max(err.values()) <= TOL and case.barriers_equal()
+    assert used > 0, "no instruction found its rows staged"
