@@ -4,6 +4,7 @@ chunk counts.  Against the CPU oracle, at the repository's bar (max-abs-rel
 2e-2, barrier tensor equal)."""
 
 import pytest
+import torch
 
 from full_harness import FullCase
 from llama_harness import LlamaCase
@@ -48,6 +49,29 @@ def test_moe_stream_sizes(hidden, ffn, experts, workers):
         # fp32 sums in another order than the oracle's flip up to 1.2 % of the
         # residuals at these sizes; a lost rounding point flips over 20 %
         case.run_token(x).assert_ok(min_exact=0.98)
+
+
+@pytest.mark.parametrize("hidden,ffn,experts", [(512, 1024, 4), (1024, 1536, 8), (1536, 1536, 16), (2560, 2048, 6),
+                                                (4608, 1024, 8)])
+def test_moe_few_items_same_bits(hidden, ffn, experts):
+    """Up to two opcode-5 items per wave go one at a time (256, 128 and 100
+    workers: 1 to 2 of them, a last round of fewer than waves), more through
+    the ring (33 and 5 workers); the bits do not depend on it, nor on work
+    sharing."""
+    seen = []
+    for workers in (256, 128, 100, 33, 5):
+        case = MoECase(MoEConfig(1, hidden, ffn, 8, 2, experts, 2, 64), seed=hidden, workers=workers,
+                       generate_on_device=True)
+        x = torch.randn(hidden, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16)
+        for kw in ({}, {"work_sharing": True}):
+            case.reset(x)
+            case.run_gpu(**kw)
+            g = case.g_gpu
+            seen.append([t.clone() for t in (g.router_normed_hidden, g.selected_expert_scores, g.expert_silu_out,
+                                             g.hidden_states)])
+    for later in seen[1:]:
+        for a, b in zip(seen[0], later):
+            assert torch.equal(a, b)
 
 
 @pytest.mark.parametrize("hidden,ffn,workers", [
