@@ -798,11 +798,15 @@ __device__ __forceinline__ int ring_fill_items(int nc) {
 // While the ring is filled (before ready()), next() is called ring_fill_items
 // times, less where the items run out: a caller whose counter is set only by
 // a barrier in ready() deals that many items itself.
-// Bound: HBM for long rows, the per-item arithmetic (sums, SiLU, claims) for
-// short ones.  Opcode 5 against one item's loads at a time (dot_pair), kernel
-// time of an MoE layer: H 2560, F 6656, 16 experts 52.5 -> 49.3 us; H 4096,
-// F 14336 122.4 -> 120.3 us; H 1024, F 3584 26.5 -> 25.7 us; H 512, F 1024
-// (one chunk, one item per wave) 20.1 -> 20.7 us.  Opcode 6 on a ring of four
+// Bound: HBM for long rows, the per-item arithmetic (sums, claims) for short
+// ones.  MoE opcode 5 with one item's loads at a time (dot_pair) -> on the
+// ring, both forms in one library, kernel time of a launch: 64 workers, H
+// 2560, F 6656 (26 items per wave) 92.7 -> 85.2 us, H 1024, F 3584 (14) 35.6
+// -> 32.7; 256 workers, H 1024, F 3584 (3.5) 28.3 -> 27.7, H 2560, F 6656
+// (6.5) 50.0 -> 49.4, H 4096, F 14336 (14) 118.5 -> 117.9.  It loses on some
+// shapes of a few items per wave, H 1536, F 4608 (4.5) 29.3 -> 30.2, H 2048,
+// F 7168 (7) 40.4 -> 41.2, H 3584, F 5120 (5) 49.0 -> 49.8, without a rule
+// that tells them from the ones it gains on.  Opcode 6 on a ring of four
 // 4-chunk slots was 1 to 8 % slower than its two 7-chunk register sets; the
 // LM heads on this ring (16 or 24 loads in flight) lost 0.7 % of eight 3B
 // layers and 2 % of a two-layer step.
@@ -927,7 +931,9 @@ __device__ __forceinline__ float lane_value(float v, int l) {
 // Reduce per-thread router partials to the E logits (+ bias): lane e of every
 // wave adds expert e's per-wave partials itself (in wave order), so the
 // logits are in registers after a single workgroup barrier, and the sums of
-// all experts take the time of one.  Returns lane e's logit.
+// all experts take the time of one (these sums and softmax_top2's exponentials
+// of all experts in every lane instead: +0.9 us at 4 experts, +1.4 to 1.7 at
+// 16, +0.7 at H 4096, F 14336, 8 experts).  Returns lane e's logit.
 template <int kE>
 __device__ __forceinline__ float finish_logits(kp_c &p, SharedState &sh, const float *acc) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1427,8 +1433,11 @@ __device__ __forceinline__ bool op_rms_router_upgate(kp_c &p, SharedState &sh, u
     // Waves take items from a workgroup counter in LDS rather than a fixed
     // stride: the memory pipeline favours older waves, so with a fixed split
     // the youngest wave ends up finishing its last items alone.  Rows of one
-    // or two chunks are the exception: the claim's LDS round trip would take
-    // as long as the item's own arithmetic.
+    // or two chunks are the exception: the claim's LDS round trip takes as
+    // long as the item's own arithmetic.  Fixed stride against claims, both in
+    // one library: H 512, F 4096 -1.1 % of the launch, H 1024, F 1536 -2.2 %,
+    // but H 1024, F 3584 +1.4 % (64 workers +1.6 %); at three chunks -1.6 and
+    // +1.7 %, at four and five +1.0 to +2.6 %.
     const bool strided = nc <= 2;
     bool started = from_lds;
     int last = wave;
@@ -1446,7 +1455,10 @@ __device__ __forceinline__ bool op_rms_router_upgate(kp_c &p, SharedState &sh, u
     };
     // An item's sums wait in one lane of (sg, su, sid) each, and up to 64 items
     // get their SiLU and their stores at once: the exponential and the
-    // division of one lane would hold up the wave's stream at every item.
+    // division of one lane would hold up the wave's stream at every item (one
+    // by one, both in one library: H 4096, F 14336 +2.5 % of the launch, H
+    // 2560, F 6656 +2.3 %, H 1024, F 3584 with 64 workers +6.1 %, one item
+    // per wave at H 512 -1 %).
     int mine = 0, held = 0, sid = 0;
     float sg = 0.f, su = 0.f;
     auto flush = [&] {
@@ -1775,7 +1787,8 @@ __device__ __forceinline__ bool op_expert_downproj(kp_c &p, SharedState &sh, u32
     // the O-projection barrier it waited for has made them final, so they
     // are read now instead of after the sums (one dependent load less; as
     // the aligned pair of rows, because a 16-bit load is followed at once by
-    // its widening, which would wait for the weights in flight too).
+    // its widening, which would wait for the weights in flight too: 0.1 us of
+    // the launch up to H 1024, nothing above).
     uint32_t hpre = 0;
     if (known && tid < first_batch) hpre = ld_dev32(p.hidden + ((row0 + tid) & ~1));
 
@@ -1787,7 +1800,7 @@ __device__ __forceinline__ bool op_expert_downproj(kp_c &p, SharedState &sh, u32
     // with ordinary (cache-allocating) loads straight into a scratch corner
     // of LDS; after the wait, their regular loads find them in the
     // Infinity Cache.  Workgroups that arrive after the last producer skip
-    // it, and their poll has been the wait.
+    // it, and their poll has been the wait (0.1 to 0.2 us of a launch).
     bool reached = false;
     if (known && p.pf_rounds > 0) {
         reached = counter_reached(p, sh, ready, expected);
@@ -3039,7 +3052,9 @@ __device__ __forceinline__ bool op_dense_upgate(kp_c &p, SharedState &sh, u32x4 
     // the wait instead, to stream while the staged items are computed, the
     // first items measured 7 % slower per decode step).  The items that the
     // fill reaches are dealt in turn, the later ones come from the LDS
-    // counter (as in the MoE's opcode 5, rows of one or two chunks excepted).
+    // counter (as in the MoE's opcode 5, rows of one or two chunks excepted;
+    // here the exception makes no difference: 0.2 % either way on eleven
+    // launches of one and two chunks, with the line at 0, 1, 2, 3 or 5).
     // Against one item ahead and then one item's loads at a time, kernel time:
     // eight 3B layers with the LM head 559.7 -> 556.4 us, one layer of H 1536,
     // F 2048 39.2 -> 38.7 us, two-layer step of H 1024 63.9 -> 63.5 us; one 3B
