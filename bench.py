@@ -57,11 +57,11 @@ HBM_PEAK_GBS = 8000.0
 # HBM bytes moved per launch (rocprofv3 FETCH_SIZE and WRITE_SIZE per
 # dispatch, each scaled by what the same counter reads for a device copy of
 # known size: FETCH x 2.0, WRITE x 1.0), measured on the kernel of commit
-# 0e3b696: config 2 one MoE layer; configs 3/4/5 one decode step at 2050 /
+# bf5ebee: config 2 one MoE layer; configs 3/4/5 one decode step at 2050 /
 # 4098 / 16386 cached positions.  The counter runs are summarised under
 # profiles/.
-MEASURED_TRAFFIC_BYTES = {"c2": 707_841_102, "c3": 6_749_136_490, "c4": 26_290_541_573, "c5": 28_033_287_742}
-TRAFFIC_UNIT = ("bytes per launch (rocprofv3 FETCH_SIZE + WRITE_SIZE, copy-calibrated, kernel of commit 0e3b696; "
+MEASURED_TRAFFIC_BYTES = {"c2": 707_493_963, "c3": 6_742_646_723, "c4": 26_280_916_773, "c5": 28_020_108_180}
+TRAFFIC_UNIT = ("bytes per launch (rocprofv3 FETCH_SIZE + WRITE_SIZE, copy-calibrated, kernel of commit bf5ebee; "
                 "configs 3-5 at 2050 / 4098 / 16386 cached positions)")
 
 
