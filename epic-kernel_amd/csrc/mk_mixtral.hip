@@ -3505,7 +3505,9 @@ __device__ __forceinline__ void exit_argmax(kp_c &p, SharedState &sh) {
         sh.flag = r.idx;
     }
     __syncthreads();
-    if (p.next_embed != nullptr) {
+    // -1: a dense launch whose schedule stored no logit (NoOps, no LM head) has
+    // no token, and no row of the table to copy
+    if (p.next_embed != nullptr && __builtin_amdgcn_readfirstlane(sh.flag) >= 0) {
         const int tok = sh.flag;
         const u32x4 *src = reinterpret_cast<const u32x4 *>(p.next_embed + (size_t)tok * p.H);
         u32x4 *dst = reinterpret_cast<u32x4 *>(p.hidden);

@@ -133,3 +133,29 @@ def test_reset_for_next_launch(dense):
         assert max_abs_rel(g.hidden_states, ref_hidden) <= 2e-2
     else:
         assert torch.equal(g.hidden_states, ref_hidden)
+
+
+@pytest.mark.parametrize("dense", [False, True], ids=["mixtral", "llama"])
+@pytest.mark.parametrize("kind", ["noops", "no_lm_head"])
+def test_launch_that_stores_no_logit(dense, kind):
+    """NoOps, or a schedule that stops before the LM head.  The Mixtral VM
+    reduces the logits as they stand (all zeros: the first); the dense one,
+    which reduces what its LM heads stored, has no token (-1) and copies no
+    embedding row."""
+    stop = "downproj" if kind == "no_lm_head" else None
+    case = LlamaCase(LLAMA_TINY, seed=4, prefill=6, stop_after_op=stop) if dense else FullCase(TINY, seed=4, prefill=6,
+                                                                                               stop_after_op=stop)
+    g, table = case.g_gpu, case.gpu_model.embed_tokens
+    if kind == "noops":
+        g.instructions.zero_()
+    out = torch.full((), -5, dtype=torch.long, device="cuda")
+    _launch(case, dense, 3, argmax_out=out)
+    left = g.hidden_states.clone()
+    _launch(case, dense, 3, argmax_out=out, next_embed_weights=table)
+    assert int(out) == (-1 if dense else 0)
+    if not dense:
+        assert torch.equal(g.hidden_states, table[0])
+    elif kind == "noops":
+        assert torch.equal(g.hidden_states, table[3])
+    else:
+        assert max_abs_rel(g.hidden_states, left) <= 2e-2  # relaunch to rounding (column chunks)
